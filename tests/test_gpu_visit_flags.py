@@ -1,0 +1,102 @@
+"""The visit flags of large fused steps come from the batch's positions
+(visit_kernel.hpp) and their hash-grid backward adds only what does not
+truncate to 0 (hash_scatter_nonzero_kernel): both against what the corners and
+the split path (flags stored by the backward) say. Marked gpu."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from test_gpu_parity import make_trainer
+from tiny_metal_nn import OptimizerStateBlob
+
+pytestmark = pytest.mark.gpu
+
+PZ = 805459861
+
+# dims, features, log2 table, levels, n: the pass's smallest batch and one
+# point to either side (131071 takes the old route), 1, 2 and 4 ranges of 2^20
+# entries, the smallest table, feature counts without a fused backward
+SHAPES = [
+    (3, 2, 19, 4, 131071), (3, 2, 19, 4, 131072), (3, 2, 19, 4, 131073), (3, 2, 10, 16, 150001),
+    (3, 4, 21, 2, 262144), (3, 1, 15, 5, 140000), (2, 2, 21, 3, 262144), (4, 2, 22, 2, 262147),
+    (4, 4, 16, 8, 131072),
+]
+
+
+def _moments(tr, value):
+    sec = [np.full(k, value, np.float32) for k in
+           (tr.hash_param_count, tr.hash_param_count, tr.mlp_param_count, tr.mlp_param_count)]
+    return OptimizerStateBlob(1, 10, b"".join(
+        np.array([4 * s.size], "<u4").tobytes() + s.tobytes() for s in sec))
+
+
+def _m_of(tr):
+    blob = tr.export_optimizer_state().payload
+    return np.frombuffer(blob, np.float32, tr.hash_param_count, 4)
+
+
+def _positions(dims, n, rng):
+    pos = rng.random((n, dims), dtype=np.float32)
+    pos[: n // 4] = pos[: n // 4] * np.float32(0.02) + np.float32(0.4)  # many points a cell
+    pos[0] = 0.0
+    pos[1] = 1.0
+    pos[2] = -0.37
+    # x cells ending in 20 one bits at resolution 16: x and x + 1 lie in
+    # different ranges of a table above 2^20 entries
+    pos[3, 0] = 65535.96875
+    pos[4] = 65535.96875
+    return pos
+
+
+@pytest.mark.parametrize("dims,feats,log2t,levels,n", SHAPES)
+def test_visited_entries_are_the_corners(dims, feats, log2t, levels, n):
+    print(f"visited set {dims}D F{feats} T2^{log2t} L{levels} n{n}", flush=True)
+    rng = np.random.default_rng(n + dims)
+    pos = _positions(dims, n, rng)
+    tgt = rng.random((n, 2), dtype=np.float32)
+    enc = dict(n_levels=levels, n_features_per_level=feats, log2_hashmap_size=log2t,
+               base_resolution=16.0, per_level_scale=2.0)
+    with make_trainer(dims, 2, enc, dict(n_neurons=64, n_hidden_layers=1), loss="L2",
+                      precision="fp16", batch=n, hash_range=0.5) as tr:
+        want = np.zeros((levels, 1 << log2t), bool)
+        for at in range(0, n, 1 << 16):
+            _, idx, _ = tr.debug_encode(pos[at:at + (1 << 16)], with_corners=True)
+            for lv in range(levels):
+                want[lv, idx[:, lv].ravel()] = True
+                if dims == 2:
+                    want[lv, idx[:, lv].ravel() ^ (PZ & ((1 << log2t) - 1))] = True
+        for _ in range(2):  # the second step's flags start from a buffer the first one cleared
+            tr.import_optimizer_state(_moments(tr, 1.0))
+            tr.training_step(pos, tgt)
+            moved = (_m_of(tr) != 1.0).reshape(levels, 1 << log2t, feats).all(axis=2)
+            assert np.array_equal(moved, want)
+
+
+@pytest.mark.parametrize("dims,feats,log2t,levels,n", [
+    (3, 2, 14, 16, 131072), (3, 4, 17, 8, 131101), (4, 2, 16, 8, 131073), (3, 1, 15, 5, 140001)])
+def test_gradients_match_the_split_path(dims, feats, log2t, levels, n):
+    """One fused step against forward_for_training, backward_accumulate (which
+    stores its flags in the backward) and adam_step: first moments within 16
+    fixed-point units times 1 - beta1, as the parity tests allow for an ulp of
+    d that moves a truncation, and exact on 99% of the entries."""
+    print(f"split parity {dims}D F{feats} T2^{log2t} L{levels} n{n}", flush=True)
+    rng = np.random.default_rng(n)
+    pos = _positions(dims, n, rng)
+    tgt = rng.random((n, 2), dtype=np.float32) * np.float32(200.0)  # large gradients
+    enc = dict(n_levels=levels, n_features_per_level=feats, log2_hashmap_size=log2t,
+               base_resolution=16.0, per_level_scale=1.5)
+    args = (dims, 2, enc, dict(n_neurons=64, n_hidden_layers=1))
+    kw = dict(loss="L2", precision="fp32", batch=n, hash_range=0.5)
+    with make_trainer(*args, **kw) as a, make_trainer(*args, **kw) as b:
+        a.import_optimizer_state(_moments(a, 0.0))
+        b.import_optimizer_state(_moments(b, 0.0))
+        a.training_step(pos, tgt)
+        out = b.forward_for_training(pos)
+        b.zero_gradients()
+        b.backward_accumulate(pos, (np.float32(2) * (out - tgt)) * np.float32(1.0 / n))
+        b.adam_step()
+        ma, mb = _m_of(a), _m_of(b)
+        assert np.count_nonzero(mb) > mb.size // 20
+        assert np.abs(ma - mb).max() <= 16 * 0.1 / 65536 + 1e-6 * np.abs(mb).max()
+        assert np.mean(ma != mb) <= 0.01

@@ -46,7 +46,7 @@ struct ScatterArgs {
   const float *pos;          // [n][D], the order dx was produced in
   const float *dx;           // [n][IN]
   int32_t *grad_hash;        // [L][T][F]
-  uint8_t *mask;             // [L][T] visit flags
+  uint8_t *mask;             // [L][T] visit flags (null: stored already, visit_kernel.hpp)
 };
 
 constexpr int kScatterThreads = 256;
@@ -232,7 +232,7 @@ __device__ __forceinline__ void scatter_level(const ScatterArgs &a, int l, const
         for (int f = 0; f < F; ++f)
           if (ci[f] != 0) atomicAdd(a.grad_hash + entry * F + f, ci[f]);
       }
-      mark_entry(a.mask, entry);
+      if (a.mask) mark_entry(a.mask, entry);
     }
   }
 }
@@ -242,9 +242,9 @@ __device__ __forceinline__ void scatter_level(const ScatterArgs &a, int l, const
 template <int D, int F>
 __device__ __forceinline__ void scatter_point_level(const ScatterArgs &a, int l, const float *p,
                                                     const float *d, bool valid, int lane) {
-  if (__all(!valid || grads_vanish<F>(d)))
-    mark_level<D, F>(a, l, p, valid);
-  else if (__all(grads_fit<F>(d)))
+  if (__all(!valid || grads_vanish<F>(d))) {
+    if (a.mask) mark_level<D, F>(a, l, p, valid);
+  } else if (__all(grads_fit<F>(d)))
     scatter_level<D, F, true>(a, l, p, d, valid, lane);
   else
     scatter_level<D, F, false>(a, l, p, d, valid, lane);

@@ -47,7 +47,8 @@ __device__ __forceinline__ void tile_scatter(const FieldArgs &a, const f32x4 (&d
   static_assert(tile_scatter_shape(D, F), "fused scatter shape");
   static_assert(0 <= GB && GB <= GE && GE <= 2 * KT0, "group range");
   const uint32_t tmask = (1u << a.log2T) - 1u;
-  const __amdgpu_buffer_rsrc_t flags = flag_rsrc(a.mask, a.L, a.log2T);
+  // no flag array: a resource of no records, which drops every store
+  const __amdgpu_buffer_rsrc_t flags = flag_rsrc(a.mask, a.mask ? a.L : 0, a.log2T);
 #pragma unroll
   for (int gi = GB; gi < GE; ++gi) {
       const int kt = gi / 2, h = gi % 2;
@@ -61,8 +62,10 @@ __device__ __forceinline__ void tile_scatter(const FieldArgs &a, const f32x4 (&d
         float d[2];
         d[0] = dx[kt][nt][2 * h] * a.inv_loss_scale;
         d[1] = dx[kt][nt][2 * h + 1] * a.inv_loss_scale;
+        const bool vanish = __all(!on || grads_vanish<2>(d));
+        if (vanish && !a.mask) continue;  // the flags are stored already (visit_kernel.hpp)
         const Cell<D> c = cell_of<D>(pos[nt], rl);
-        if (__all(!on || grads_vanish<2>(d))) {
+        if (vanish) {
           // flags only. Corners x and x + 1 of a cell differ only in the low
           // bits the carry of x + 1 flips, so their flag bytes share a
           // 128-byte line unless x ends in seven 1 bits: one

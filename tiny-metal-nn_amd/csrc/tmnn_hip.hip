@@ -33,6 +33,7 @@
 #include "scatter_kernel.hpp"
 #include "sort.hpp"
 #include "step_kernel.hpp"
+#include "visit_kernel.hpp"
 #include "wide_kernel.hpp"
 #include "wide_train_kernel.hpp"
 
@@ -288,6 +289,7 @@ struct tmnn_trainer {
   tmnn_network_plan plan{};
 
   DevBuf params, m, v, grad_hash, grad_mlp;
+  DevBuf visit_bits;  // visit_kernel's bits, one set per share of the batch
   DevBuf mask[2];  // visit flags, double-buffered: Adam reads one, zeroes the other
   int mask_cur = 0;
   DevBuf partials, loss_partials, loss_out;
@@ -310,6 +312,9 @@ struct tmnn_trainer {
   hipStream_t side = nullptr;
   hipEvent_t ev_sorted[kSortSets] = {};
   hipEvent_t ev_consumed[kSortSets] = {};
+  hipEvent_t ev_flags_free = nullptr;  // the flag buffer is zeroed (visit pass may start)
+  hipEvent_t ev_visited = nullptr;     // the visit pass of the step being enqueued
+  bool visit_pending = false;          // the finish kernel has to wait for ev_visited
   hipEvent_t ev_staged = nullptr;  // host-staged batch copied in on the main stream
   bool consumed_recorded[kSortSets] = {};
   int sort_parity = 0;
@@ -372,7 +377,8 @@ struct tmnn_trainer {
     for (int k = 0; k < kSortSets; ++k)
       for (hipEvent_t e : {ev_sorted[k], ev_consumed[k]})
         if (e) (void)hipEventDestroy(e);
-    if (ev_staged) (void)hipEventDestroy(ev_staged);
+    for (hipEvent_t e : {ev_staged, ev_flags_free, ev_visited})
+      if (e) (void)hipEventDestroy(e);
     for (KernelPlan *p : {&train_plan, &fwd_plan, &infer_plan, &grad_plan})
       if (p->image) (void)hipFree(p->image);
     for (auto &set : prof_events)
@@ -1285,7 +1291,7 @@ int sort_batch(tmnn_trainer *tr, const float *d_pos, const float *d_tgt,
 
 // Hash-grid backward of the dx the train kernel left in tr->dx for the n
 // points at pos (same order): table gradients + visit flags.
-int launch_scatter(tmnn_trainer *tr, const float *pos, int n) {
+int launch_scatter(tmnn_trainer *tr, const float *pos, int n, bool flags_apart) {
   ScatterArgs s{};
   s.n = n;
   s.IN = tr->IN;
@@ -1294,7 +1300,27 @@ int launch_scatter(tmnn_trainer *tr, const float *pos, int n) {
   s.pos = pos;
   s.dx = tr->dx.as<float>();
   s.grad_hash = tr->grad_hash.as<int32_t>();
-  s.mask = tr->mask[tr->mask_cur].as<uint8_t>();
+  s.mask = flags_apart ? nullptr : tr->mask[tr->mask_cur].as<uint8_t>();
+  if (flags_apart) {
+    const dim3 groups((n + kNonzeroPoints - 1) / kNonzeroPoints);
+#define TMNN_NONZERO(d, f)                                                              \
+  launch_step_kernel(tr, kKernScatter, hash_scatter_nonzero_kernel<d, f>, groups,       \
+                     dim3(kScatterThreads), 0, tr->ctx->stream, s)
+    switch (tr->d.spatial_dims * 8 + tr->d.features_per_level) {
+      case 2 * 8 + 1: TMNN_NONZERO(2, 1); break;
+      case 2 * 8 + 2: TMNN_NONZERO(2, 2); break;
+      case 2 * 8 + 4: TMNN_NONZERO(2, 4); break;
+      case 3 * 8 + 1: TMNN_NONZERO(3, 1); break;
+      case 3 * 8 + 2: TMNN_NONZERO(3, 2); break;
+      case 3 * 8 + 4: TMNN_NONZERO(3, 4); break;
+      case 4 * 8 + 1: TMNN_NONZERO(4, 1); break;
+      case 4 * 8 + 2: TMNN_NONZERO(4, 2); break;
+      default: TMNN_NONZERO(4, 4); break;
+    }
+#undef TMNN_NONZERO
+    TMNN_HIP_TRY(hipGetLastError());
+    return TMNN_OK;
+  }
   // point-major while a level's slice of the table is cache-sized, else
   // level-major (one level's slice at a time). Point-major 3D splits a
   // point's levels over four threads (C3: 415 -> 378 us); 2D keeps one
@@ -1327,6 +1353,84 @@ int launch_scatter(tmnn_trainer *tr, const float *pos, int n) {
   return TMNN_OK;
 }
 
+// Sparse hash Adam needs l1_reg == 0 (default_trainer.cpp:1868-1876).
+bool lazy_adam(const tmnn_trainer *tr) {
+  return tr->d.hash_adam_mode == TMNN_HASH_ADAM_LAZY && tr->d.l1_reg == 0.0f;
+}
+
+// Whether a fused step of n points takes its visit flags from the positions
+// (visit_kernel) instead of from the hash-grid backward. Steps without / with
+// the pass, us (3D 16x2: 2^17 points 118 / 115 at T = 2^15, 199 / 184 at 2^19,
+// 2^18 points 275 / 224 at 2^19; 3D 16x4, 2^17 points 348 / 313 at 2^19; 4D
+// 16x2, 2^18 points 417 / 308 at 2^15, 1479 / 1178 at 2^22): below 2^17 points
+// the two extra launches cost what they save (2^16 points 109 / 117 at 3D
+// 2^17, 158 / 162 at 4D 2^17). 2D points have half the corners of 3D ones and
+// their flags stay in the L2s up to large tables: 88 / 94 at 2^15, 149 / 150
+// at 2^19, but 386 / 369 (2^18 points) and 885 / 617 (2^20) at 2^21.
+bool visit_pass(const tmnn_trainer *tr, int n) {
+  if (!lazy_adam(tr)) return false;
+  // a pass over the table's bits for too few points (2^18 points and T = 2^24: 1783 / 1815)
+  if ((static_cast<uint64_t>(n) << (tr->d.spatial_dims + 1)) >> tr->d.log2_hashmap_size == 0)
+    return false;
+  if (tr->d.spatial_dims == 2) return n >= (1 << 18) && tr->d.log2_hashmap_size >= 21;
+  return n >= (1 << 17);
+}
+
+using VisitKernel = void (*)(VisitArgs);
+
+VisitKernel visit_kernel_of(int dims, bool ranged) {
+  switch (dims) {
+    case 2: return ranged ? visit_kernel<2, true> : visit_kernel<2, false>;
+    case 3: return ranged ? visit_kernel<3, true> : visit_kernel<3, false>;
+    default: return ranged ? visit_kernel<4, true> : visit_kernel<4, false>;
+  }
+}
+
+// The pass over n points: one block per CU (two, where the bits leave room,
+// read 43 us instead of 57 at 2^20 3D points and T = 2^19, but cost the encode
+// they run beside more: step 507 us instead of 496).
+struct VisitShape {
+  uint32_t log2W, lds, rows, shares;
+};
+
+VisitShape visit_shape(const tmnn_trainer *tr, int n) {
+  VisitShape s{};
+  const uint32_t log2T = static_cast<uint32_t>(tr->d.log2_hashmap_size);
+  s.log2W = std::min(log2T, kVisitLog2Range) - 5u;
+  s.lds = 4u << s.log2W;
+  s.rows = static_cast<uint32_t>(tr->d.num_levels) << (log2T - s.log2W - 5u);
+  const uint32_t most = (static_cast<uint32_t>(n) + kVisitThreads - 1u) / kVisitThreads;
+  s.shares = std::max(1u, std::min(most, static_cast<uint32_t>(tr->ctx->cu_count) / s.rows));
+  return s;
+}
+
+// The visit flags of n points at pos, on stream st.
+int launch_visit(tmnn_trainer *tr, const float *pos, int n, hipStream_t st) {
+  const VisitShape s = visit_shape(tr, n);
+  VisitArgs v{};
+  v.n = n;
+  v.share = static_cast<int32_t>((static_cast<uint32_t>(n) + s.shares - 1u) / s.shares);
+  v.log2T = static_cast<uint32_t>(tr->d.log2_hashmap_size);
+  v.log2W = s.log2W;
+  for (int l = 0; l < kMaxLevels; ++l) v.res[l] = tr->res[l];
+  v.pos = pos;
+  v.bits = tr->visit_bits.as<uint32_t>();
+  hipLaunchKernelGGL(visit_kernel_of(tr->d.spatial_dims, v.log2T > s.log2W + 5u),
+                     dim3(s.shares, s.rows), dim3(kVisitThreads), s.lds, st, v);
+  TMNN_HIP_TRY(hipGetLastError());
+  VisitExpandArgs x{};
+  x.bits = v.bits;
+  x.total = s.rows << s.log2W;
+  x.log2W = s.log2W;
+  x.shares = static_cast<int32_t>(s.shares);
+  x.mask = tr->mask[tr->mask_cur].as<uint8_t>();
+  hipLaunchKernelGGL(visit_expand_kernel,
+                     dim3((x.total + kVisitExpandThreads - 1u) / kVisitExpandThreads),
+                     dim3(kVisitExpandThreads), 0, st, x);
+  TMNN_HIP_TRY(hipGetLastError());
+  return TMNN_OK;
+}
+
 // Flags of the events that order the side stream's sort and the main stream's
 // step. Both streams run on this device, so the producer's release and the
 // consumer's acquire only need device scope: without
@@ -1341,9 +1445,19 @@ constexpr unsigned kSyncEventFlags = hipEventDisableTiming | hipEventDisableSyst
 // was staged on the main stream, for that copy); the main stream then waits
 // for the sort. The caller marks the set consumed after the step
 // (sort_set_consumed). Returns the permutation in *perm_out.
+// visit: the side stream then also takes the batch's visit flags
+// (visit_kernel), once the main stream is done with what was enqueued before
+// this step (the last finish kernel zeroes the flag buffer); the finish
+// kernel waits for them (ev_visited). The pass is VALU- and LDS-bound and
+// runs beside the memory-bound encode.
 int sort_batch_overlapped(tmnn_trainer *tr, const float *d_pos, int n, bool staged_on_main,
-                          const uint32_t **perm_out) {
+                          bool visit, const uint32_t **perm_out) {
   hipStream_t st = tr->ctx->stream;
+  if (visit) {
+    for (hipEvent_t *e : {&tr->ev_flags_free, &tr->ev_visited})
+      if (!*e) TMNN_HIP_TRY(hipEventCreateWithFlags(e, kSyncEventFlags));
+    TMNN_HIP_TRY(hipEventRecord(tr->ev_flags_free, st));
+  }
   if (!tr->side) {
     TMNN_HIP_TRY(hipStreamCreateWithFlags(&tr->side, hipStreamNonBlocking));
     for (int k = 0; k < tmnn_trainer::kSortSets; ++k) {
@@ -1371,6 +1485,13 @@ int sort_batch_overlapped(tmnn_trainer *tr, const float *d_pos, int n, bool stag
                                  &sorted_keys, perm_out));
   TMNN_HIP_TRY(hipEventRecord(tr->ev_sorted[k], sd));
   TMNN_HIP_TRY(hipStreamWaitEvent(st, tr->ev_sorted[k], 0));
+  if (visit) {
+    TMNN_HIP_TRY(hipStreamWaitEvent(sd, tr->ev_flags_free, 0));
+    const int rc = launch_visit(tr, d_pos, n, sd);
+    if (rc != TMNN_OK) return rc;
+    TMNN_HIP_TRY(hipEventRecord(tr->ev_visited, sd));
+    tr->visit_pending = true;
+  }
   return TMNN_OK;
 }
 
@@ -1398,10 +1519,12 @@ int run_forward_backward(tmnn_trainer *tr, const float *d_pos, const float *d_tg
   if (rc != TMNN_OK) return rc;
   // the packed weight image (rebuilt after every Adam step) counts with the sort
   if ((rc = ensure_image(tr, tr->train_plan)) != TMNN_OK) return rc;
+  const bool visit = !reduce && visit_pass(tr, n);
   if (overlap_sort && tr->d.morton_sort && n > 1 && tr->train_plan.xmem) {
     // feature-tile plans read the batch through the permutation (no gather)
-    rc = sort_batch_overlapped(tr, d_pos, n, overlap_sort > 1, &perm);
+    rc = sort_batch_overlapped(tr, d_pos, n, overlap_sort > 1, visit, &perm);
   } else {
+    if (visit && (rc = launch_visit(tr, d_pos, n, tr->ctx->stream)) != TMNN_OK) return rc;
     rc = sort_batch(tr, d_pos, d_tgt, tr->d.num_outputs, n, &pos, &tgt, &perm,
                     !tr->train_plan.xmem);
   }
@@ -1431,13 +1554,13 @@ int run_forward_backward(tmnn_trainer *tr, const float *d_pos, const float *d_tg
   if (fused_scatter) {  // the training kernel runs the hash-grid backward per tile
     a.spos = indexed ? sorted_pos : pos;
     a.grad_hash = tr->grad_hash.as<int32_t>();
-    a.mask = tr->mask[tr->mask_cur].as<uint8_t>();
+    a.mask = visit ? nullptr : tr->mask[tr->mask_cur].as<uint8_t>();
   }
   const int blocks = launch_field(tr, tr->train_plan, a, n, 2, false, a.tgt_index, sorted_pos);
   if (blocks < 0) return blocks;
   if ((rc = prof_mark(tr, 3)) != TMNN_OK) return rc;
   if (!fused_scatter) {  // else the scatter phase is empty (no boundary event)
-    if ((rc = launch_scatter(tr, indexed ? sorted_pos : pos, n)) != TMNN_OK) return rc;
+    if ((rc = launch_scatter(tr, indexed ? sorted_pos : pos, n, visit)) != TMNN_OK) return rc;
     if ((rc = prof_mark(tr, 4)) != TMNN_OK) return rc;
   }
   if (!reduce) return blocks;  // finish_step_kernel reduces the rows and the loss
@@ -1458,8 +1581,7 @@ AdamArgs adam_args(tmnn_trainer *tr, bool clear_grads, bool clear_mask) {
   a.v = tr->v.as<float>();
   a.grad_hash = tr->grad_hash.as<int32_t>();
   a.grad_mlp = tr->grad_mlp.as<float>();
-  // Sparse hash Adam needs l1_reg == 0 (default_trainer.cpp:1868-1876).
-  a.lazy = (tr->d.hash_adam_mode == TMNN_HASH_ADAM_LAZY && tr->d.l1_reg == 0.0f) ? 1 : 0;
+  a.lazy = lazy_adam(tr) ? 1 : 0;
   a.mask = tr->mask[tr->mask_cur].as<uint8_t>();
   a.mask_next = tr->mask[tr->mask_cur ^ 1].as<uint8_t>();
   a.partner_xor = tr->d.spatial_dims == 2 ? (kPrimeZ & ((1u << tr->d.log2_hashmap_size) - 1u)) : 0u;
@@ -1664,6 +1786,10 @@ int train_step_device(tmnn_trainer *tr, const float *d_pos, const float *d_tgt, 
     prof_abort(tr);
     if (overlapped) (void)sort_set_consumed(tr);
     return blocks;
+  }
+  if (tr->visit_pending) {
+    tr->visit_pending = false;
+    TMNN_HIP_TRY(hipStreamWaitEvent(tr->ctx->stream, tr->ev_visited, 0));
   }
   // dW reduction, loss and Adam in one kernel (the reduce phase is empty: no
   // boundary event)
@@ -2019,6 +2145,15 @@ int tmnn_trainer_create(tmnn_context *ctx, const tmnn_model_desc *desc, tmnn_tra
   if ((rc = plan_kernel(tr.get(), tr->d.precision == TMNN_PRECISION_FP16, true,
                         tr->train_plan)) != TMNN_OK)
     return rc;
+  if (visit_pass(tr.get(), desc->batch_size)) {
+    const VisitShape vs = visit_shape(tr.get(), desc->batch_size);
+    TMNN_HIP_TRY(tr->visit_bits.ensure(static_cast<size_t>(vs.shares) * (tr->hash_entries / 8u)));
+    const int log2R = std::min<int>(desc->log2_hashmap_size, kVisitLog2Range);
+    TMNN_HIP_TRY(hipFuncSetAttribute(
+        reinterpret_cast<const void *>(
+            visit_kernel_of(desc->spatial_dims, desc->log2_hashmap_size > log2R)),
+        hipFuncAttributeMaxDynamicSharedMemorySize, 1 << (log2R - 3)));
+  }
   if ((rc = plan_kernel(tr.get(), tr->d.precision == TMNN_PRECISION_FP16, false,
                         tr->fwd_plan)) != TMNN_OK)
     return rc;
