@@ -1684,6 +1684,31 @@ int run_finish(tmnn_trainer *tr, int part_blocks, int n, float *d_loss) {
   return TMNN_OK;
 }
 
+// The position gradients of one output from tr->dx.
+int launch_pos_grad(tmnn_trainer *tr, const PosGradArgs &g) {
+  int log2L = 0;
+  while ((1 << log2L) < g.L) ++log2L;
+  const int points = kPosGradThreads >> log2L;
+  const dim3 grid((static_cast<uint32_t>(g.n) + points - 1) / points);
+#define TMNN_POS_GRAD(d, f)                                                                  \
+  hipLaunchKernelGGL((pos_grad_kernel<d, f>), grid, dim3(kPosGradThreads), 0, tr->ctx->stream, \
+                     g, log2L)
+  switch (tr->d.spatial_dims * 8 + tr->d.features_per_level) {
+    case 2 * 8 + 1: TMNN_POS_GRAD(2, 1); break;
+    case 2 * 8 + 2: TMNN_POS_GRAD(2, 2); break;
+    case 2 * 8 + 4: TMNN_POS_GRAD(2, 4); break;
+    case 3 * 8 + 1: TMNN_POS_GRAD(3, 1); break;
+    case 3 * 8 + 2: TMNN_POS_GRAD(3, 2); break;
+    case 3 * 8 + 4: TMNN_POS_GRAD(3, 4); break;
+    case 4 * 8 + 1: TMNN_POS_GRAD(4, 1); break;
+    case 4 * 8 + 2: TMNN_POS_GRAD(4, 2); break;
+    default: TMNN_POS_GRAD(4, 4); break;
+  }
+#undef TMNN_POS_GRAD
+  TMNN_HIP_TRY(hipGetLastError());
+  return TMNN_OK;
+}
+
 int zero_device(tmnn_trainer *tr, void *ptr, size_t bytes) {
   if (bytes == 0) return TMNN_OK;
   const size_t n16 = (bytes + 15) / 16;
@@ -2475,13 +2500,7 @@ int tmnn_evaluate_with_gradient(tmnn_trainer *tr, const float *positions, float 
     const int blocks = launch_field(tr, tr->grad_plan, a, n, -1, m > 0);
     if (blocks < 0) return blocks;
     g.m = m;
-    const dim3 grid((n + 255) / 256);
-    switch (tr->d.spatial_dims) {
-      case 2: hipLaunchKernelGGL(pos_grad_kernel<2>, grid, dim3(256), 0, st, g); break;
-      case 3: hipLaunchKernelGGL(pos_grad_kernel<3>, grid, dim3(256), 0, st, g); break;
-      default: hipLaunchKernelGGL(pos_grad_kernel<4>, grid, dim3(256), 0, st, g); break;
-    }
-    TMNN_HIP_TRY(hipGetLastError());
+    if ((rc = launch_pos_grad(tr, g)) != TMNN_OK) return rc;
   }
   TMNN_HIP_TRY(hipMemcpyAsync(output, tr->out_buf.ptr, n * M * sizeof(float),
                               hipMemcpyDeviceToHost, st));
