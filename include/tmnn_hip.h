@@ -112,7 +112,8 @@ typedef struct tmnn_model_desc {
   int32_t batch_size;         /* steps use min(N, batch_size) points */
   int32_t precision;          /* TMNN_PRECISION_* (training / split path) */
   int32_t hash_adam_mode;     /* TMNN_HASH_ADAM_* */
-  int32_t morton_sort;        /* 1: sort each batch by Morton code (reference) */
+  int32_t morton_sort;        /* 1: batches whose order pays are sorted by Morton code (the
+                                 reference sorts every batch); 0: none is */
   /* weight init */
   uint64_t seed;
   float hash_init_range;      /* U(-r, r) for the table */

@@ -47,8 +47,8 @@ __device__ __forceinline__ void tile_scatter(const FieldArgs &a, const f32x4 (&d
   static_assert(tile_scatter_shape(D, F), "fused scatter shape");
   static_assert(0 <= GB && GB <= GE && GE <= 2 * KT0, "group range");
   const uint32_t tmask = (1u << a.log2T) - 1u;
-  // no flag array: a resource of no records, which drops every store
-  const __amdgpu_buffer_rsrc_t flags = flag_rsrc(a.mask, a.mask ? a.L : 0, a.log2T);
+  // no flag array (3D): a resource of no records, which drops every store
+  const __amdgpu_buffer_rsrc_t flags = flag_rsrc(a.mask, D == 2 || a.mask ? a.L : 0, a.log2T);
 #pragma unroll
   for (int gi = GB; gi < GE; ++gi) {
       const int kt = gi / 2, h = gi % 2;
@@ -63,7 +63,8 @@ __device__ __forceinline__ void tile_scatter(const FieldArgs &a, const f32x4 (&d
         d[0] = dx[kt][nt][2 * h] * a.inv_loss_scale;
         d[1] = dx[kt][nt][2 * h + 1] * a.inv_loss_scale;
         const bool vanish = __all(!on || grads_vanish<2>(d));
-        if (vanish && !a.mask) continue;  // the flags are stored already (visit_kernel.hpp)
+        if constexpr (D == 3)  // 2D tables of this kernel's sizes never take the visit pass
+          if (vanish && !a.mask) continue;  // the flags come from visit_kernel
         const Cell<D> c = cell_of<D>(pos[nt], rl);
         if (vanish) {
           // flags only. Corners x and x + 1 of a cell differ only in the low

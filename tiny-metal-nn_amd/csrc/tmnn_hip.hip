@@ -1217,27 +1217,44 @@ float loss_scale_for(int n, bool f16) {
   return std::ldexp(1.0f, std::min(e, 24));
 }
 
-int ensure_batch(tmnn_trainer *tr, int n) {
+// Whether a batch is put in Morton order at all: where its order saves more
+// gather and scatter time than the sort's kernels (twelve in 3D and 4D, four
+// in 2D, on a second stream in the fused device step) and their events cost.
+// Steps sorted / unsorted, us: 3D 16x2 T = 2^19 2^16 points 158 / 143, 2^17
+// 181 / 164, 2^18 223 / 220; 3D 16x4 T = 2^19 264 / 254, 314 / 306, 408 / 416;
+// 4D 16x2 T = 2^19 316 / 288, 417 / 371, 611 / 589; a synchronous 16-wide step
+// of 4096 points 152 / 71. 2D 16x2 T = 2^15: 2^14 points 51 / 40, 2^16
+// 49 / 51, 2^17 61 / 68, 2^18 87 / 109. From 2^17 points on the order also
+// keeps the visit pass (visit_pass) beside the sort. Results differ by the
+// order of their fp32 sums only.
+bool sorts(const tmnn_trainer *tr, int n) {
+  return tr->d.morton_sort && n > (tr->d.spatial_dims == 2 ? 1 << 15 : (1 << 17) - 1);
+}
+
+// Buffers of a batch of n points (order: those of its sort too).
+int ensure_batch(tmnn_trainer *tr, int n, bool order) {
   const size_t D = tr->d.spatial_dims, M = tr->d.num_outputs;
   TMNN_HIP_TRY(tr->in_pos.ensure(n * D * sizeof(float)));
   TMNN_HIP_TRY(tr->in_tgt.ensure(n * M * sizeof(float)));
-  TMNN_HIP_TRY(tr->s_pos.ensure(n * D * sizeof(float)));
-  TMNN_HIP_TRY(tr->s_tgt.ensure(n * M * sizeof(float)));
-  TMNN_HIP_TRY(tr->keys0.ensure(n * sizeof(uint32_t)));
-  TMNN_HIP_TRY(tr->keys1.ensure(n * sizeof(uint32_t)));
-  TMNN_HIP_TRY(tr->vals0.ensure(n * sizeof(uint32_t)));
-  TMNN_HIP_TRY(tr->vals1.ensure(n * sizeof(uint32_t)));
-  size_t tmp = 0;
-  TMNN_HIP_TRY(morton_sort_temp_bytes(n, &tmp));
-  TMNN_HIP_TRY(tr->sort_tmp.ensure(std::max<size_t>(tmp, 256)));
-  if (tr->d.morton_sort)
-    for (auto &ss : tr->step_sort) {
-      TMNN_HIP_TRY(ss.keys0.ensure(n * sizeof(uint32_t)));
-      TMNN_HIP_TRY(ss.keys1.ensure(n * sizeof(uint32_t)));
-      TMNN_HIP_TRY(ss.vals0.ensure(n * sizeof(uint32_t)));
-      TMNN_HIP_TRY(ss.vals1.ensure(n * sizeof(uint32_t)));
-      TMNN_HIP_TRY(ss.tmp.ensure(std::max<size_t>(tmp, 256)));
-    }
+  if (order) {
+    TMNN_HIP_TRY(tr->s_pos.ensure(n * D * sizeof(float)));
+    TMNN_HIP_TRY(tr->s_tgt.ensure(n * M * sizeof(float)));
+    TMNN_HIP_TRY(tr->keys0.ensure(n * sizeof(uint32_t)));
+    TMNN_HIP_TRY(tr->keys1.ensure(n * sizeof(uint32_t)));
+    TMNN_HIP_TRY(tr->vals0.ensure(n * sizeof(uint32_t)));
+    TMNN_HIP_TRY(tr->vals1.ensure(n * sizeof(uint32_t)));
+    size_t tmp = 0;
+    TMNN_HIP_TRY(morton_sort_temp_bytes(n, &tmp));
+    TMNN_HIP_TRY(tr->sort_tmp.ensure(std::max<size_t>(tmp, 256)));
+    if (tr->d.morton_sort)
+      for (auto &ss : tr->step_sort) {
+        TMNN_HIP_TRY(ss.keys0.ensure(n * sizeof(uint32_t)));
+        TMNN_HIP_TRY(ss.keys1.ensure(n * sizeof(uint32_t)));
+        TMNN_HIP_TRY(ss.vals0.ensure(n * sizeof(uint32_t)));
+        TMNN_HIP_TRY(ss.vals1.ensure(n * sizeof(uint32_t)));
+        TMNN_HIP_TRY(ss.tmp.ensure(std::max<size_t>(tmp, 256)));
+      }
+  }
   // dx rows for the whole last tile: the MLP train kernel stores unconditionally
   TMNN_HIP_TRY(tr->dx.ensure(static_cast<size_t>((n + kTilePts - 1) / kTilePts) * kTilePts *
                              tr->IN * sizeof(float)));
@@ -1253,14 +1270,16 @@ int ensure_batch(tmnn_trainer *tr, int n) {
 }
 
 // Morton order of the batch: returns the permutation (sorted i -> original
-// row), or nullptr when sorting is off. With gather, also the sorted copies
+// row), or nullptr when sorting is off or does not pay (always: the inspection
+// entries ask for the order itself). With gather, also the sorted copies
 // of (pos, tgt) in s_pos / s_tgt (else *pos_out / *tgt_out are the inputs:
 // the training path reads them through the permutation).
 int sort_batch(tmnn_trainer *tr, const float *d_pos, const float *d_tgt,
                int tgt_dims, int n, const float **pos_out,
-               const float **tgt_out, const uint32_t **perm_out, bool gather = true) {
+               const float **tgt_out, const uint32_t **perm_out, bool gather = true,
+               bool always = false) {
   hipStream_t st = tr->ctx->stream;
-  if (!tr->d.morton_sort || n <= 1) {
+  if (!sorts(tr, n) && !(always && tr->d.morton_sort && n > 1)) {
     *pos_out = d_pos;
     *tgt_out = d_tgt;
     *perm_out = nullptr;
@@ -1520,7 +1539,7 @@ int run_forward_backward(tmnn_trainer *tr, const float *d_pos, const float *d_tg
   // the packed weight image (rebuilt after every Adam step) counts with the sort
   if ((rc = ensure_image(tr, tr->train_plan)) != TMNN_OK) return rc;
   const bool visit = !reduce && visit_pass(tr, n);
-  if (overlap_sort && tr->d.morton_sort && n > 1 && tr->train_plan.xmem) {
+  if (overlap_sort && sorts(tr, n) && tr->train_plan.xmem) {
     // feature-tile plans read the batch through the permutation (no gather)
     rc = sort_batch_overlapped(tr, d_pos, n, overlap_sort > 1, visit, &perm);
   } else {
@@ -1801,7 +1820,7 @@ int train_step_device(tmnn_trainer *tr, const float *d_pos, const float *d_tgt, 
   int rc = prof_begin_step(tr);
   if (rc != TMNN_OK) return rc;
   float *loss = d_loss ? d_loss : tr->loss_out.as<float>();
-  const bool overlapped = overlap_sort && tr->d.morton_sort && n > 1 && tr->train_plan.xmem;
+  const bool overlapped = overlap_sort && sorts(tr, n) && tr->train_plan.xmem;
   tr->num_this_step = num;
   tr->input_ready = input_ready;
   const int blocks = run_forward_backward(tr, d_pos, d_tgt, n, false, loss, false, overlap_sort);
@@ -1922,7 +1941,7 @@ int host_training_step(tmnn_trainer *tr, const float *input, const float *target
   if (!input || !target) return fail(TMNN_ERR_INVALID_ARGUMENT, "input/target is null");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   const int bn = std::min(n, tr->d.batch_size);
-  int rc = ensure_batch(tr, bn);
+  int rc = ensure_batch(tr, bn, sorts(tr, bn));
   if (rc != TMNN_OK) return rc;
   hipStream_t st = tr->ctx->stream;
   const size_t M = tr->d.num_outputs;
@@ -2265,7 +2284,7 @@ int tmnn_training_step_device_after(tmnn_trainer *tr, const float *d_input,
   if (!d_input || !d_target) return fail(TMNN_ERR_INVALID_ARGUMENT, "input/target is null");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   const int bn = std::min(n, tr->d.batch_size);
-  const int rc = ensure_batch(tr, bn);
+  const int rc = ensure_batch(tr, bn, sorts(tr, bn));
   if (rc != TMNN_OK) return rc;
   // device steps are sampled by step only: their losses are not read back
   return train_step_device(tr, d_input, d_target, bn, d_loss_out, 1,
@@ -2470,7 +2489,7 @@ int tmnn_evaluate_with_gradient(tmnn_trainer *tr, const float *positions, float 
   }
   hipStream_t st = tr->ctx->stream;
   const size_t D = tr->d.spatial_dims, M = tr->d.num_outputs;
-  if ((rc = ensure_batch(tr, n)) != TMNN_OK) return rc;
+  if ((rc = ensure_batch(tr, n, false)) != TMNN_OK) return rc;
   TMNN_HIP_TRY(tr->out_buf.ensure(n * M * sizeof(float)));
   TMNN_HIP_TRY(tr->grad_out.ensure(n * M * D * sizeof(float)));
   TMNN_HIP_TRY(hipMemcpyAsync(tr->in_pos.ptr, positions, n * D * sizeof(float),
@@ -2519,7 +2538,7 @@ int tmnn_forward_for_training(tmnn_trainer *tr, const float *input, float *outpu
   if (!input || !output) return fail(TMNN_ERR_INVALID_ARGUMENT, "input/output is null");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   const int bn = std::min(n, tr->d.batch_size);
-  int rc = ensure_batch(tr, bn);
+  int rc = ensure_batch(tr, bn, sorts(tr, bn));
   if (rc != TMNN_OK) return rc;
   hipStream_t st = tr->ctx->stream;
   const size_t D = tr->d.spatial_dims, M = tr->d.num_outputs;
@@ -2560,7 +2579,7 @@ int tmnn_backward_accumulate(tmnn_trainer *tr, const float *input, const float *
   if (!input || !d_output) return fail(TMNN_ERR_INVALID_ARGUMENT, "input/d_output is null");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   const int bn = std::min(n, tr->d.batch_size);
-  int rc = ensure_batch(tr, bn);
+  int rc = ensure_batch(tr, bn, sorts(tr, bn));
   if (rc != TMNN_OK) return rc;
   hipStream_t st = tr->ctx->stream;
   TMNN_HIP_TRY(hipMemcpyAsync(tr->in_pos.ptr, input,
@@ -2937,7 +2956,7 @@ int tmnn_debug_encode_tiles(tmnn_trainer *tr, const float *positions, int32_t n,
   if (!positions || !features) return fail(TMNN_ERR_INVALID_ARGUMENT, "null argument");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   hipStream_t st = tr->ctx->stream;
-  int rc = ensure_batch(tr, n);
+  int rc = ensure_batch(tr, n, true);
   if (rc != TMNN_OK) return rc;
   const size_t D = tr->d.spatial_dims;
   TMNN_HIP_TRY(hipMemcpyAsync(tr->in_pos.ptr, positions, n * D * sizeof(float),
@@ -2945,7 +2964,7 @@ int tmnn_debug_encode_tiles(tmnn_trainer *tr, const float *positions, int32_t n,
   const float *pos = tr->in_pos.as<float>(), *unused = nullptr;
   const uint32_t *perm = nullptr;
   if (sorted) {
-    rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, n, &pos, &unused, &perm, false);
+    rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, n, &pos, &unused, &perm, false, true);
     if (rc != TMNN_OK) return rc;
   }
   float *pos_out = perm ? tr->s_pos.as<float>() : nullptr;
@@ -2984,11 +3003,12 @@ int tmnn_debug_hash_rates(tmnn_trainer *tr, const float *d_positions, int32_t n,
   if (n <= 0 || reps < 1) return fail(TMNN_ERR_INVALID_ARGUMENT, "N and reps must be >= 1");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   hipStream_t st = tr->ctx->stream;
-  int rc = ensure_batch(tr, n);
+  int rc = ensure_batch(tr, n, true);
   if (rc != TMNN_OK) return rc;
   const float *pos = d_positions, *unused = nullptr;
   const uint32_t *perm = nullptr;
-  if (sorted && (rc = sort_batch(tr, d_positions, nullptr, 0, n, &pos, &unused, &perm)) != TMNN_OK)
+  if (sorted && (rc = sort_batch(tr, d_positions, nullptr, 0, n, &pos, &unused, &perm, true, true)) !=
+                    TMNN_OK)
     return rc;
   TMNN_HIP_TRY(tr->dbg_a.ensure(static_cast<size_t>(tr->hash_count) * sizeof(int32_t)));
   TMNN_HIP_TRY(tr->dbg_b.ensure(tr->hash_entries));
@@ -3164,7 +3184,7 @@ int tmnn_debug_morton_sort(tmnn_trainer *tr, const float *positions, int32_t n, 
   if (!positions || !codes || !perm) return fail(TMNN_ERR_INVALID_ARGUMENT, "null argument");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   hipStream_t st = tr->ctx->stream;
-  int rc = ensure_batch(tr, n);
+  int rc = ensure_batch(tr, n, true);
   if (rc != TMNN_OK) return rc;
   const size_t D = tr->d.spatial_dims;
   TMNN_HIP_TRY(hipMemcpyAsync(tr->in_pos.ptr, positions, n * D * sizeof(float),
@@ -3178,7 +3198,7 @@ int tmnn_debug_morton_sort(tmnn_trainer *tr, const float *positions, int32_t n, 
   TMNN_HIP_TRY(hipStreamSynchronize(st));
   const float *sp = nullptr, *stg = nullptr;
   const uint32_t *p = nullptr;
-  rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, n, &sp, &stg, &p);
+  rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, n, &sp, &stg, &p, true, true);
   if (rc != TMNN_OK) return rc;
   if (!p && n == 1) {
     perm[0] = 0u;  // a single point is its own order
