@@ -293,6 +293,23 @@ __global__ void zero_bytes_kernel(uint8_t *dst, size_t n) {
     dst[i] = 0;
 }
 
+// Two buffers in 16-byte pieces, between a context's pinned staging memory and
+// device memory (both allocated in multiples of 256 bytes).
+struct StageCopyArgs {
+  const uint4 *src[2];
+  uint4 *dst[2];
+  uint32_t pieces[2];
+};
+constexpr int kStageThreads = 256;
+
+__global__ void __launch_bounds__(kStageThreads) stage_copy_kernel(StageCopyArgs a) {
+  const uint32_t i = blockIdx.x * kStageThreads + threadIdx.x;
+  if (i < a.pieces[0])
+    a.dst[0][i] = a.src[0][i];
+  else if (i - a.pieces[0] < a.pieces[1])
+    a.dst[1][i - a.pieces[0]] = a.src[1][i - a.pieces[0]];
+}
+
 // Encode-only inspection kernel: thread per (point, level).
 template <int D>
 __device__ void encode_debug_point(const float *table, uint32_t log2T, int F,
