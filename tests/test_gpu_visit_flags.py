@@ -14,12 +14,12 @@ pytestmark = pytest.mark.gpu
 
 PZ = 805459861
 
-# dims, features, log2 table, levels, n: the pass's smallest batch and one
-# point to either side (131071 takes the old route), 1, 2 and 4 ranges of 2^20
-# entries, the smallest table, feature counts without a fused backward
+# dims, features, log2 table, levels, n: the pass's smallest batch at T = 2^19
+# and one point to either side (131071 takes the other route), 1, 2 and 4 ranges
+# of 2^20 entries, the smallest table, feature counts without a fused backward
 SHAPES = [
-    (3, 2, 19, 4, 131071), (3, 2, 19, 4, 131072), (3, 2, 19, 4, 131073), (3, 2, 10, 16, 150001),
-    (3, 4, 21, 2, 262144), (3, 1, 15, 5, 140000), (2, 2, 21, 3, 262144), (4, 2, 22, 2, 262147),
+    (3, 2, 19, 4, 131071), (3, 2, 19, 4, 131072), (3, 2, 19, 4, 131073), (3, 2, 10, 16, 524289),
+    (3, 4, 21, 2, 262144), (3, 1, 15, 5, 262145), (2, 2, 21, 3, 262144), (4, 2, 22, 2, 262147),
     (4, 4, 16, 8, 131072),
 ]
 
@@ -74,7 +74,7 @@ def test_visited_entries_are_the_corners(dims, feats, log2t, levels, n):
 
 
 @pytest.mark.parametrize("dims,feats,log2t,levels,n", [
-    (3, 2, 14, 16, 131072), (3, 4, 17, 8, 131101), (4, 2, 16, 8, 131073), (3, 1, 15, 5, 140001)])
+    (3, 2, 14, 16, 524288), (3, 4, 17, 8, 262149), (4, 2, 16, 8, 131073), (3, 1, 15, 5, 262201)])
 def test_gradients_match_the_split_path(dims, feats, log2t, levels, n):
     """One fused step against forward_for_training, backward_accumulate (which
     stores its flags in the backward) and adam_step: first moments within 16

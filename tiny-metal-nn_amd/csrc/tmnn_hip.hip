@@ -28,6 +28,7 @@
 #include "field_kernel.hpp"
 #include "grad_kernel.hpp"
 #include "layer_kernels.hpp"
+#include "layer_split_kernel.hpp"
 #include "rate_kernels.hpp"
 #include "mlp_kernel.hpp"
 #include "scatter_kernel.hpp"
@@ -1111,6 +1112,16 @@ int launch_layerwise(tmnn_trainer *tr, KernelPlan &plan, FieldArgs a, int n,
       TMNN_HIP_TRY(hipGetLastError());
       return TMNN_OK;
     }
+    if (lw_split_ok(g)) {
+      int t_c = 0;
+      if (const LwGemmFn fn = lw_split_fn(g, chunks, tr->ctx->cu_count, &t_c)) {
+        const int rows = g.R - (g.ones_row ? 1 : 0);
+        const dim3 grid((rows + kLsRows - 1) / kLsRows, (g.C + t_c - 1) / t_c, chunks);
+        hipLaunchKernelGGL(fn, grid, dim3(256), 0, st, g);
+        TMNN_HIP_TRY(hipGetLastError());
+        return TMNN_OK;
+      }
+    }
     const dim3 grid((g.R + kLwTile - 1) / kLwTile, (g.C + kLwTile - 1) / kLwTile, chunks);
     const LwGemmFn fn = lw_gemm_fn(g);
     if (!fn) return fail(TMNN_ERR_RUNTIME, "layer-wise product of an unexpected form");
@@ -1469,20 +1480,23 @@ bool lazy_adam(const tmnn_trainer *tr) {
 
 // Whether a fused step of n points takes its visit flags from the positions
 // (visit_kernel) instead of from the hash-grid backward. Steps without / with
-// the pass, us (3D 16x2: 2^17 points 118 / 115 at T = 2^15, 199 / 184 at 2^19,
-// 2^18 points 275 / 224 at 2^19; 3D 16x4, 2^17 points 348 / 313 at 2^19; 4D
-// 16x2, 2^18 points 417 / 308 at 2^15, 1479 / 1178 at 2^22): below 2^17 points
-// the two extra launches cost what they save (2^16 points 109 / 117 at 3D
-// 2^17, 158 / 162 at 4D 2^17). 2D points have half the corners of 3D ones and
-// their flags stay in the L2s up to large tables: 88 / 94 at 2^15, 149 / 150
-// at 2^19, but 386 / 369 (2^18 points) and 885 / 617 (2^20) at 2^21.
+// the pass, us. 4D 16x2: 2^17 points 365 / 331 at T = 2^16, 1214 / 1082 at
+// 2^22; 2^16 points 158 / 162. 3D, T >= 2^19: 2^17 points 199 / 184 (16x2),
+// 348 / 313 (16x4). Below, 3D kernels that run their own backward hide the
+// flag stores behind the MLP up to 2^18 points (355 / 364 in fp32, 198 / 202
+// in fp16 at T = 2^16; 2^19 points 603 / 568 and 336 / 299), the separate
+// backward up to 2^17 (114 / 118; 2^18 points 186 / 177). 2D points have half
+// the corners of 3D ones and their flags stay in the L2s up to large tables:
+// 88 / 94 at 2^15, 149 / 150 at 2^19, but 386 / 369 (2^18 points) and 885 /
+// 617 (2^20) at 2^21.
 bool visit_pass(const tmnn_trainer *tr, int n) {
   if (!lazy_adam(tr)) return false;
-  // a pass over the table's bits for too few points (2^18 points and T = 2^24: 1783 / 1815)
-  if ((static_cast<uint64_t>(n) << (tr->d.spatial_dims + 1)) >> tr->d.log2_hashmap_size == 0)
-    return false;
-  if (tr->d.spatial_dims == 2) return n >= (1 << 18) && tr->d.log2_hashmap_size >= 21;
-  return n >= (1 << 17);
+  const int log2T = tr->d.log2_hashmap_size, dims = tr->d.spatial_dims;
+  // a pass over the table's bits for too few points (3D, 2^18 points, T = 2^24: 1783 / 1815)
+  if ((static_cast<uint64_t>(n) << (dims + 1)) >> log2T == 0) return false;
+  if (dims == 2) return n >= (1 << 18) && log2T >= 21;
+  if (dims == 4 || log2T >= 19) return n >= (1 << 17);
+  return n >= (tr->train_plan.tile_scatter ? 1 << 19 : 1 << 18);
 }
 
 using VisitKernel = void (*)(VisitArgs);
