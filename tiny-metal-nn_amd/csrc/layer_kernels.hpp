@@ -8,7 +8,8 @@
 // KernelSpec shape (kernel_spec.cpp:12-44) runs.
 //
 // Products: C[r][c] = sum_k A(r, k) B(k, c) over 64 x 64 output tiles (row
-// tiles along blockIdx.x, column tiles along blockIdx.y), K in steps of 16
+// tiles along blockIdx.x, column tiles along blockIdx.y; products with at
+// least 96 K and aligned rows run on layer_split_kernel.hpp instead), K in steps of 16
 // staged through LDS, each of the block's four waves a 32 x 32 quadrant on
 // the matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands, fp32
 // accumulation). The

@@ -7,9 +7,10 @@
 // free), products of bf16 values are exact in fp32, and of the nine partial
 // products the three dropped ones (m l, l m, l l) are below 2^-25 of the
 // product: six v_mfma_f32_16x16x32_bf16 per 32 K replace eight fp32 MFMAs at
-// 6/16 of their time. The leading products have an accumulator of their own:
-// rounded once per 32 K instead of eight times, it ends closer to 64 bits than
-// the fp32 MFMAs (all six in one accumulator ended 5 to 50% further off). Non-finite operands give non-finite results
+// 6/16 of their time. The running accumulator takes a step's leading product
+// and the sum of the five smaller ones: two roundings per 32 K where the fp32
+// MFMAs round eight times, and results closer to 64 bits than theirs (with all
+// six products on the running accumulator they ended 5 to 50% further off). Non-finite operands give non-finite results
 // (an infinity may come out as NaN).
 //
 // Tile: 64 x TC outputs (TC 64 or 128) per 256-thread block, each of its four
@@ -19,7 +20,9 @@
 // as 64 x 128 at 65536 x 256 x 256 and slower everywhere below. The
 // weights' side is the MFMA's row operand, so that a lane ends up with four
 // consecutive columns of one output row: 16-byte epilogue accesses without a
-// pass through LDS.
+// pass through LDS. 65536 x 256 x 256: forward 101 -> 69 us, delta 104 -> 64,
+// weight gradient 131 -> 76 (the fp32 MFMA tiles ran at 82 to 85 TFLOP/s), the
+// h256_3d step 534 -> 405 us.
 #pragma once
 
 #include "layer_kernels.hpp"
@@ -67,7 +70,9 @@ __device__ __forceinline__ int ls_slot(int row, int q) {
 // Global side of an operand tile: T rows by 32 K from (r0, k0), NQ quads of
 // four floats per thread. KFAST: K contiguous in memory (quad: four K of one
 // row; eight lanes read a row's 128 bytes). Else rows contiguous (quad: four
-// rows at one K; T / 4 lanes read one K's T rows).
+// rows at one K; neighbouring lanes take neighbouring K, so that a 16-lane
+// store covers whole rows of the LDS planes; lanes along the rows met four to a
+// bank: the 257 x 256 weight gradient of 65536 points 84 us against 76).
 template <int T, bool KFAST>
 struct LsOperand {
   static constexpr int NQ = T / 32;  // quads per thread
@@ -80,8 +85,8 @@ struct LsOperand {
     const int t = threadIdx.x;
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
-      const int r = r0 + (KFAST ? t / 8 + 32 * i : 4 * (t % kRowQuads));
-      const int k = k0 + (KFAST ? 4 * (t % 8) : (t / kRowQuads) * NQ + i);
+      const int r = r0 + (KFAST ? t / 8 + 32 * i : 4 * (t / kGroups));
+      const int k = k0 + (KFAST ? 4 * (t % 8) : (t % kGroups) * NQ + i);
       // the host checked that rows (row-fast) or K (K-fast) is a multiple of 4
       const bool in = r < rows && k < ke;
       const size_t at = KFAST ? static_cast<size_t>(in ? r : 0) * ld + (in ? k : 0)
@@ -105,7 +110,7 @@ struct LsOperand {
         *reinterpret_cast<uint2 *>(d + 2 * plane) = make_uint2(a.l, b.l);
       }
     } else {
-      const int row0 = 4 * (t % kRowQuads), k = (t / kRowQuads) * NQ;
+      const int row0 = 4 * (t / kGroups), k = (t % kGroups) * NQ;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         unsigned char *d = S + ls_slot<T>(row0 + e, k >> 3) + 2 * (k & 7);
@@ -126,7 +131,7 @@ struct LsOperand {
 };
 
 template <int TC, int AM, int BT, int EPI>
-__global__ void __launch_bounds__(256, TC == 128 ? 3 : 4) lw_split_kernel(LwGemmArgs g) {
+__global__ void __launch_bounds__(256, 4) lw_split_kernel(LwGemmArgs g) {
   constexpr int TR = kLsRows;
   constexpr bool kAKFast = AM == kLwARow;
   constexpr int kAPlane = TR * 64, kBPlane = TC * 64;
@@ -141,11 +146,11 @@ __global__ void __launch_bounds__(256, TC == 128 ? 3 : 4) lw_split_kernel(LwGemm
   const int rows = g.R - (g.ones_row ? 1 : 0);
   const int kb = blockIdx.z * g.k_chunk;
   const int ke = min(g.K, kb + g.k_chunk);
-  f32x4 acc[MR][MC], low[MR][MC];  // h h; the five smaller products
+  f32x4 acc[MR][MC];
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
-    for (int j = 0; j < MC; ++j) acc[i][j] = low[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < MC; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   LsOperand<TR, kAKFast> a;
   LsOperand<TC, BT != 0> b;
   // bias gradients (ones_row): the column sums of B, by the first row of blocks
@@ -178,32 +183,27 @@ __global__ void __launch_bounds__(256, TC == 128 ? 3 : 4) lw_split_kernel(LwGemm
 #pragma unroll
       for (int s = 0; s < 3; ++s)
         af[i][s] = *reinterpret_cast<const bf16x8 *>(As + s * kAPlane + ls_slot<TR>(wr + 16 * i + p, q));
-    // column tiles in pairs: four independent accumulators between two MFMAs
-    // on one
 #pragma unroll
-    for (int j0 = 0; j0 < MC; j0 += 2) {
-      bf16x8 bf[2][3];
+    for (int j = 0; j < MC; ++j) {
+      bf16x8 bf[3];
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int s = 0; s < 3; ++s)
-          bf[j][s] = *reinterpret_cast<const bf16x8 *>(
-              Bs + s * kBPlane + ls_slot<TC>(wc + 16 * (j0 + j) + p, q));
+      for (int s = 0; s < 3; ++s)
+        bf[s] = *reinterpret_cast<const bf16x8 *>(Bs + s * kBPlane + ls_slot<TC>(wc + 16 * j + p, q));
+      // a step's five smaller products from zero, smallest first
       constexpr int kSmall[5][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}};
+      f32x4 low[MR];
 #pragma unroll
       for (int t = 0; t < 5; ++t)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int i = 0; i < MR; ++i)
-            low[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                bf[j][kSmall[t][0]], af[i][kSmall[t][1]], low[i][j0 + j], 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
         for (int i = 0; i < MR; ++i)
-          acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j][0], af[i][0],
-                                                                   acc[i][j0 + j], 0, 0, 0);
+          low[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              bf[kSmall[t][0]], af[i][kSmall[t][1]], t == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : low[i], 0,
+              0, 0);
+#pragma unroll
+      for (int i = 0; i < MR; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[0], af[i][0], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < MR; ++i) acc[i][j] += low[i];
     }
     __syncthreads();
     if (more) {
@@ -221,7 +221,7 @@ __global__ void __launch_bounds__(256, TC == 128 ? 3 : 4) lw_split_kernel(LwGemm
     for (int j = 0; j < MC; ++j) {
       const int c = c0 + wc + 16 * j + 4 * q;
       if (c >= g.C) continue;
-      f32x4 o = acc[i][j] + low[i][j];
+      f32x4 o = acc[i][j];
       if constexpr (EPI == kLwEpiHidden) {
         const f32x4 bias = *reinterpret_cast<const f32x4 *>(g.bias + c);
 #pragma unroll
@@ -246,16 +246,16 @@ __global__ void __launch_bounds__(256, TC == 128 ? 3 : 4) lw_split_kernel(LwGemm
   }
   if constexpr (EPI == kLwEpiPartial) {
     if (!sums) return;  // uniform over the block
-    // threads t % kRowQuads share four columns; groups in ascending order
+    // threads t / kGroups share four columns; K groups in ascending order
     constexpr int kQuads = TC / 4, kGroups = 256 / kQuads;
     f32x4 *red = reinterpret_cast<f32x4 *>(smem);
     __syncthreads();
     red[tid] = colsum;
     __syncthreads();
     if (tid < kQuads && c0 + 4 * tid < g.C) {
-      f32x4 t = red[tid];
+      f32x4 t = red[tid * kGroups];
 #pragma unroll
-      for (int k = 1; k < kGroups; ++k) t += red[k * kQuads + tid];
+      for (int k = 1; k < kGroups; ++k) t += red[tid * kGroups + k];
       float *dst = g.dst + blockIdx.z * g.dst_stride + g.dst_off +
                    static_cast<int64_t>(rows) * g.C + c0 + 4 * tid;
 #pragma unroll
