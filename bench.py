@@ -192,7 +192,8 @@ def median_phases(samples) -> dict:
 
 def kernel_rooflines(phase_us: dict, models: dict, names: dict, n: int, fused_scatter: bool,
                      mlp_shape: tuple, lds_peak_gbs: float, rates: dict | None,
-                     traffic: dict | None = None, fp32: bool = False) -> list[dict]:
+                     traffic: dict | None = None, fp32: bool = False,
+                     flags_apart: bool = False) -> list[dict]:
     """Roofline entries of one training step's kernels from the kernels'
     median durations (phase_us): encode and finish (Adam) against the HBM
     peak (the encode also against its gather-only reference kernel); the MLP
@@ -201,7 +202,10 @@ def kernel_rooflines(phase_us: dict, models: dict, names: dict, n: int, fused_sc
     backward it runs in its tiles (fused_scatter) rated against the
     flag-store-only reference kernel at the same shape; a separate scatter
     kernel against its flag and atomic references. mlp_shape = (kernel's
-    input width, hidden layers, waves per block)."""
+    input width, hidden layers, waves per block). flags_apart: the step takes
+    its visit flags from the positions (visit_kernel, on the second stream),
+    so neither backward stores any: a separate one is rated by the dx it has
+    to read, a fused one not at all."""
     out = []
     mfma_peak = FP32_MFMA_PEAK_TFLOPS if fp32 else MFMA_F16_PEAK_TFLOPS
     for key, phase, kern in (("encode", "gpu_encode_us", "gpu_encode_kernel_us"),
@@ -245,7 +249,7 @@ def kernel_rooflines(phase_us: dict, models: dict, names: dict, n: int, fused_sc
                     r.update({"bound": "mfma", "achieved": mfma["achieved"], "peak": mfma_peak,
                               "unit": "TFLOP/s", "frac": round(t_mfma / us, 4)})
                 r["roofline_us"] = round(max(t_mfma, t_lds), 2)
-            if fused_scatter and rates:
+            if fused_scatter and rates and not flags_apart:
                 sb = models["scatter_fused"]["per_point"] * n
                 t_ref = rates["flag_us"]
                 r["fused_scatter"] = {
@@ -264,7 +268,7 @@ def kernel_rooflines(phase_us: dict, models: dict, names: dict, n: int, fused_sc
                 r["achievable"] = {"reference": "gather-only kernel (the encode's corner loads)",
                                    "us": round(rates["gather_us"], 2),
                                    "frac_of_achievable": round(rates["gather_us"] / us, 4)}
-            if rates and key == "scatter":
+            if rates and key == "scatter" and not flags_apart:
                 r["achievable"] = {"reference": "flag-store-only and atomic-only kernels",
                                    "flag_us": round(rates["flag_us"], 2),
                                    "atomic_us": round(rates["atomic_us"], 2)}
@@ -494,15 +498,18 @@ def run_workload(torch, which: str, steps: int, warmup: int, lds_peak_gbs: float
     models = kernel_models(d, levels, feats, m, inp, hidden, nhl, levels * feats << log2t,
                            mlp_params)
     lm = which in ("c3", "c4", "c5")
+    # 3D and 4D batches of this size take their visit flags from the positions
+    if lm:
+        models["scatter"] = {"bound": "hbm", "per_point": 4 * levels * feats}
     names = {"encode": f"encode_level_kernel<{d}, {feats}>" if lm
              else f"encode_features_kernel<{d}, {feats}>",
              "mlp": mlp_kernel_name(which, fused, precision),
-             "scatter": f"hash_scatter_level_kernel<{d}, {feats}>" if lm
+             "scatter": f"hash_scatter_nonzero_kernel<{d}, {feats}>" if lm
              else f"hash_scatter_kernel<{d}, {feats}>",
              "adam": f"finish_step_kernel<{feats}, false>"}
     ph = median_phases(samples)
     per_kernel = kernel_rooflines(ph, models, names, n, fused, (inp, nhl, ins["waves_per_block_train"]),
-                                  lds_peak_gbs, rates, fp32=precision == "fp32")
+                                  lds_peak_gbs, rates, fp32=precision == "fp32", flags_apart=lm)
     return {"workload": which, "precision": precision, "batch": n,
             "encoding": f"{d}D L{levels} F{feats} T2^{log2t} base{base:g} x{scale:g}",
             "mlp": f"{inp}->{hidden}x{nhl}->{m}", "loss": loss,
