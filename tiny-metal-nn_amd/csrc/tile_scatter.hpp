@@ -62,10 +62,10 @@ __device__ __forceinline__ void tile_scatter(const FieldArgs &a, const f32x4 (&d
         float d[2];
         d[0] = dx[kt][nt][2 * h] * a.inv_loss_scale;
         d[1] = dx[kt][nt][2 * h + 1] * a.inv_loss_scale;
+        const Cell<D> c = cell_of<D>(pos[nt], rl);
         const bool vanish = __all(!on || grads_vanish<2>(d));
         if constexpr (D == 3)  // 2D tables of this kernel's sizes never take the visit pass
           if (vanish && !a.mask) continue;  // the flags come from visit_kernel
-        const Cell<D> c = cell_of<D>(pos[nt], rl);
         if (vanish) {
           // flags only. Corners x and x + 1 of a cell differ only in the low
           // bits the carry of x + 1 flips, so their flag bytes share a
