@@ -62,3 +62,82 @@ def test_forward_error_against_64_bits(width, n):
             if i < 3:
                 x = np.maximum(x, 0)
         assert np.linalg.norm(out - x) <= 4e-7 * np.linalg.norm(x)
+
+
+def _forward64(mw, sizes, x):
+    """The MLP in 64 bits with the path's ReLU (a NaN gives 0)."""
+    at, acts = 0, [x]
+    for i, (a, b) in enumerate(zip(sizes, sizes[1:])):
+        w = mw[at:at + a * b].reshape(a, b).astype(np.float64)
+        x = x @ w + mw[at + a * b:at + a * b + b]
+        at += a * b + b
+        if i < len(sizes) - 2:
+            x = np.where(x > 0, x, 0.0)
+        acts.append(x)
+    return acts
+
+
+def _same(got, want, tol):
+    """Equal where infinite or NaN, within tol of |want| + rms elsewhere."""
+    got, want = np.asarray(got, np.float64), np.asarray(want, np.float64)
+    kinds = (np.isnan, np.isposinf, np.isneginf)
+    for kind in kinds:
+        assert np.array_equal(kind(got), kind(want)), kind.__name__
+    fin = np.isfinite(want)
+    if fin.any():
+        rms = np.sqrt((want[fin] ** 2).mean())
+        assert np.all(np.abs(got[fin] - want[fin]) <= tol * (np.abs(want[fin]) + rms))
+
+
+# an infinite entry of W_0 makes a hidden unit's activations infinite; one of
+# W_1 is itself an operand of the split product
+@pytest.mark.parametrize("layer,value", [
+    (0, np.inf), (1, np.inf), (1, -np.inf), (1, 3.4e38), (1, -3.4e38)])
+@pytest.mark.parametrize("width,n", [(256, 200), (96, 65)])
+def test_values_without_bf16_parts(width, n, layer, value):
+    """Infinities and finite values above bf16's largest (3.39e38) keep their
+    fp32 meaning: outputs and weight gradients are infinite, NaN and finite
+    where 64 bits says so, and a step over infinite outputs reports a loss that
+    is not finite. The finite rest within 1e-5, the repository's fp32 bar."""
+    print(f"split products without parts w{width} layer {layer} {value}", flush=True)
+    rng = np.random.default_rng(width + layer)
+    sizes = [16, width, width, 2]
+    at = [0, 17 * width, (17 + width + 1) * width]
+    with make_trainer(3, 2, ENC, dict(n_neurons=width, n_hidden_layers=2), hash_range=0.5,
+                      batch=n) as tr, np.errstate(all="ignore"):
+        hw, mw = (w.copy() for w in tr.get_weights())
+        hw = np.abs(hw)  # positive features: an infinite W_0[0][unit] reaches every point
+        if np.isfinite(value):
+            hw *= np.float32(1e-3)  # hidden activations below 1, so that 3.4e38 times them is finite
+        tr.set_initial_weights(hw, mw)
+        pos = rng.random((n, 3), dtype=np.float32)
+        feats = tr.debug_encode(pos).astype(np.float64)
+        unit = int(np.argmax((_forward64(mw, sizes, feats)[1] > 0).sum(0)))
+        if layer == 0:
+            mw[unit] = value
+            row = at[1] + unit * width  # W_1's row of that unit: values whose lower parts are 0
+            mw[row:row + width] = np.where(rng.random(width) < 0.5, 0.25, -0.25)
+        else:
+            mw[at[1] + unit * width + 3] = value
+        tr.set_initial_weights(hw, mw)
+        acts = _forward64(mw, sizes, feats)
+        if np.isfinite(value):
+            assert np.abs(acts[2]).max() < 3.4e38
+        _same(tr.inference(pos), acts[-1], 1e-5)
+        if np.isfinite(value):
+            return
+        d = rng.normal(0, 1.0, (n, 2)).astype(np.float32)
+        tr.zero_gradients()
+        tr.backward_accumulate(pos, d)
+        _, gm = tr.debug_gradients()
+        want, d = [], d.astype(np.float64)
+        for i in (2, 1, 0):
+            a, b = sizes[i], sizes[i + 1]
+            want.append(np.concatenate([(acts[i].T @ d).ravel(), d.sum(0)]))
+            d = d @ mw[at[i]:at[i] + a * b].reshape(a, b).astype(np.float64).T
+            if i:
+                d = np.where(acts[i] > 0, d, 0.0)
+        _same(gm, np.concatenate(want[::-1]), 1e-5)
+        finite = np.isfinite(acts[-1]).all()
+        assert finite == (value < 0)
+        assert np.isfinite(tr.training_step(pos, np.zeros((n, 2), np.float32))) == finite

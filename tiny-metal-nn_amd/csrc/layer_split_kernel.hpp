@@ -10,8 +10,11 @@
 // 6/16 of their time. The running accumulator takes a step's leading product
 // and the sum of the five smaller ones: two roundings per 32 K where the fp32
 // MFMAs round eight times, and results closer to 64 bits than theirs (with all
-// six products on the running accumulator they ended 5 to 50% further off). Non-finite operands give non-finite results
-// (an infinity may come out as NaN).
+// six products on the running accumulator they ended 5 to 50% further off).
+// An infinity or a value above bf16's largest (3.39e38) has no such parts: its
+// products are NaN. An output whose sum is not finite is computed again in
+// fp32 before its epilogue (ls_exact), whose ReLU would otherwise turn that
+// NaN into 0.
 //
 // Tile: 64 x TC outputs (TC 64 or 128) per 256-thread block, each of its four
 // waves a quarter, K in steps of 32 whose split planes sit in LDS. The split's
@@ -130,6 +133,32 @@ struct LsOperand {
   }
 };
 
+__device__ __forceinline__ bool ls_finite(float v) {
+  return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u;
+}
+
+// Outputs (r, c .. c + 3) over K in [kb, ke): where the split sum in o is not
+// finite, the sum of the fp32 products instead. Finite sums had finite parts
+// and stay. Rare, so its loop is small rather than fast.
+template <int AM, int BT>
+__device__ __forceinline__ f32x4 ls_exact(const LwGemmArgs &g, int r, int c, int kb, int ke,
+                                          f32x4 o) {
+  bool keep[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) keep[e] = ls_finite(o[e]);
+  if (keep[0] && keep[1] && keep[2] && keep[3]) return o;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int k = kb; k < ke; ++k) {
+    const float a = lw_a<AM>(g, r, k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = __builtin_fmaf(a, lw_b<BT>(g, k, c + e), s[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) s[e] = keep[e] ? o[e] : s[e];
+  return s;
+}
+
 template <int TC, int AM, int BT, int EPI>
 __global__ void __launch_bounds__(256, 4) lw_split_kernel(LwGemmArgs g) {
   constexpr int TR = kLsRows;
@@ -221,7 +250,7 @@ __global__ void __launch_bounds__(256, 4) lw_split_kernel(LwGemmArgs g) {
     for (int j = 0; j < MC; ++j) {
       const int c = c0 + wc + 16 * j + 4 * q;
       if (c >= g.C) continue;
-      f32x4 o = acc[i][j];
+      f32x4 o = ls_exact<AM, BT>(g, r, c, kb, ke, acc[i][j]);
       if constexpr (EPI == kLwEpiHidden) {
         const f32x4 bias = *reinterpret_cast<const f32x4 *>(g.bias + c);
 #pragma unroll
