@@ -1318,18 +1318,54 @@ float loss_scale_for(int n, bool f16) {
   return std::ldexp(1.0f, std::min(e, 24));
 }
 
+// What a batch is put in Morton order for.
+enum SortPass {
+  kSortForward,   // a forward pass only
+  kSortHostPass,  // a host-pointer step or backward: the sort is waited for
+  kSortDeviceStep // a device-pointer step: the sort runs beside the previous step
+};
+
 // Whether a batch is put in Morton order at all: where its order saves more
 // gather and scatter time than the sort's kernels (twelve in 3D and 4D, four
 // in 2D, on a second stream in the fused device step) and their events cost.
+// Results differ by the order of their fp32 sums only.
+//
+// Forward passes, and training kernels that run the hash-grid backward
+// themselves (tile_scatter: no merging across lanes, so the order only moves
+// the gathers), leave batches unsorted up to 2^17 - 1 points (2^15 in 2D).
 // Steps sorted / unsorted, us: 3D 16x2 T = 2^19 2^16 points 158 / 143, 2^17
-// 181 / 164, 2^18 223 / 220; 3D 16x4 T = 2^19 264 / 254, 314 / 306, 408 / 416;
-// 4D 16x2 T = 2^19 316 / 288, 417 / 371, 611 / 589; a synchronous 16-wide step
-// of 4096 points 152 / 71. 2D 16x2 T = 2^15: 2^14 points 51 / 40, 2^16
-// 49 / 51, 2^17 61 / 68, 2^18 87 / 109. From 2^17 points on the order also
-// keeps the visit pass (visit_pass) beside the sort. Results differ by the
-// order of their fp32 sums only.
-bool sorts(const tmnn_trainer *tr, int n) {
-  return tr->d.morton_sort && n > (tr->d.spatial_dims == 2 ? 1 << 15 : (1 << 17) - 1);
+// 181 / 164, 2^18 223 / 220; 2D 16x2 T = 2^15: 2^14 points 51 / 40, 2^16
+// 49 / 51, 2^17 61 / 68, 2^18 87 / 109; positions spread over 1 to 1/500 of
+// the domain and gradients small to large: 1.05 to 1.15 in the mean, 0.91 at
+// worst. From 2^17 points on the order also keeps the visit pass (visit_pass)
+// beside the sort.
+//
+// The separate hash-grid backward merges the runs of lanes that share an entry
+// (scatter_kernel.hpp), which only a sorted batch has: without them clustered
+// points meet in the atomics (sorted / unsorted, us: 3D 8x4 T = 2^17 131071
+// points over 1/50 of the domain 1618 / 11803, 3D 8x2 32768 186 / 803, 2D 8x2
+// 8192 86 / 235, spread ones 3D 8x2 131071 387 / 599). It is left out only up
+// to the sizes where even that costs no more than the sort does, at worst
+// 0.95 over those spreads and gradients: host passes 16x2 T = 2^17: 3D 4096
+// points 157 / 89 spread, 173 / 181 clustered (8192: 196 / 273), 2D 2048
+// 152 / 100, 137 / 139 (4096: 154 / 185), 4D 8192 201 / 121, 524 / 479; device
+// steps 3D 1024 69 / 52, 79 / 76 (2048: 83 / 104), 4D 8192 106 / 92, 437 / 448,
+// none in 2D (512: 69 / 82). Four features (16x4) add by four 32-bit atomics
+// and lose in 2D and 3D at once (3D 1024: host 212 / 235, device 135 / 211).
+bool sorts(const tmnn_trainer *tr, int n, SortPass pass) {
+  if (!tr->d.morton_sort || n <= 1) return false;
+  const int dims = tr->d.spatial_dims;
+  if (pass == kSortForward || tr->train_plan.tile_scatter)
+    return n > (dims == 2 ? 1 << 15 : (1 << 17) - 1);
+  if (dims == 4) return n > 8192;
+  if (tr->d.features_per_level == 4) return true;
+  if (pass == kSortHostPass) return n > (dims == 2 ? 2048 : 4096);
+  return dims == 2 || n > 1024;
+}
+
+// The pass of a step by train_step_device's overlap_sort (2: a host batch).
+SortPass step_sort_pass(int overlap_sort) {
+  return overlap_sort == 2 ? kSortHostPass : kSortDeviceStep;
 }
 
 // Buffers of a batch of n points (order: those of its sort too).
@@ -1370,17 +1406,16 @@ int ensure_batch(tmnn_trainer *tr, int n, bool order) {
   return TMNN_OK;
 }
 
-// Morton order of the batch: returns the permutation (sorted i -> original
-// row), or nullptr when sorting is off or does not pay (always: the inspection
-// entries ask for the order itself). With gather, also the sorted copies
-// of (pos, tgt) in s_pos / s_tgt (else *pos_out / *tgt_out are the inputs:
+// Morton order of the batch where order says so (sorts; the inspection entries
+// ask for the order itself): returns the permutation (sorted i -> original
+// row), else nullptr. With gather, also the sorted copies of (pos, tgt) in
+// s_pos / s_tgt (else *pos_out / *tgt_out are the inputs:
 // the training path reads them through the permutation).
 int sort_batch(tmnn_trainer *tr, const float *d_pos, const float *d_tgt,
                int tgt_dims, int n, const float **pos_out,
-               const float **tgt_out, const uint32_t **perm_out, bool gather = true,
-               bool always = false) {
+               const float **tgt_out, const uint32_t **perm_out, bool order, bool gather = true) {
   hipStream_t st = tr->ctx->stream;
-  if (!sorts(tr, n) && !(always && tr->d.morton_sort && n > 1)) {
+  if (!order) {
     *pos_out = d_pos;
     *tgt_out = d_tgt;
     *perm_out = nullptr;
@@ -1643,12 +1678,13 @@ int run_forward_backward(tmnn_trainer *tr, const float *d_pos, const float *d_tg
   // the packed weight image (rebuilt after every Adam step) counts with the sort
   if ((rc = ensure_image(tr, tr->train_plan)) != TMNN_OK) return rc;
   const bool visit = !reduce && visit_pass(tr, n);
-  if (overlap_sort && sorts(tr, n) && tr->train_plan.xmem) {
+  const bool order = sorts(tr, n, external_grad ? kSortHostPass : step_sort_pass(overlap_sort));
+  if (overlap_sort && order && tr->train_plan.xmem) {
     // feature-tile plans read the batch through the permutation (no gather)
     rc = sort_batch_overlapped(tr, d_pos, n, overlap_sort > 1, visit, &perm);
   } else {
     if (visit && (rc = launch_visit(tr, d_pos, n, tr->ctx->stream)) != TMNN_OK) return rc;
-    rc = sort_batch(tr, d_pos, d_tgt, tr->d.num_outputs, n, &pos, &tgt, &perm,
+    rc = sort_batch(tr, d_pos, d_tgt, tr->d.num_outputs, n, &pos, &tgt, &perm, order,
                     !tr->train_plan.xmem);
   }
   if (rc != TMNN_OK) return rc;
@@ -1924,7 +1960,8 @@ int train_step_device(tmnn_trainer *tr, const float *d_pos, const float *d_tgt, 
   int rc = prof_begin_step(tr);
   if (rc != TMNN_OK) return rc;
   float *loss = d_loss ? d_loss : tr->loss_out.as<float>();
-  const bool overlapped = overlap_sort && sorts(tr, n) && tr->train_plan.xmem;
+  const bool overlapped =
+      overlap_sort && sorts(tr, n, step_sort_pass(overlap_sort)) && tr->train_plan.xmem;
   tr->num_this_step = num;
   tr->input_ready = input_ready;
   const int blocks = run_forward_backward(tr, d_pos, d_tgt, n, false, loss, false, overlap_sort);
@@ -2045,7 +2082,7 @@ int host_training_step(tmnn_trainer *tr, const float *input, const float *target
   if (!input || !target) return fail(TMNN_ERR_INVALID_ARGUMENT, "input/target is null");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   const int bn = std::min(n, tr->d.batch_size);
-  int rc = ensure_batch(tr, bn, sorts(tr, bn));
+  int rc = ensure_batch(tr, bn, sorts(tr, bn, kSortHostPass));
   if (rc != TMNN_OK) return rc;
   hipStream_t st = tr->ctx->stream;
   const size_t M = tr->d.num_outputs;
@@ -2400,7 +2437,7 @@ int tmnn_training_step_device_after(tmnn_trainer *tr, const float *d_input,
   if (!d_input || !d_target) return fail(TMNN_ERR_INVALID_ARGUMENT, "input/target is null");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   const int bn = std::min(n, tr->d.batch_size);
-  const int rc = ensure_batch(tr, bn, sorts(tr, bn));
+  const int rc = ensure_batch(tr, bn, sorts(tr, bn, kSortDeviceStep));
   if (rc != TMNN_OK) return rc;
   // device steps are sampled by step only: their losses are not read back
   return train_step_device(tr, d_input, d_target, bn, d_loss_out, 1,
@@ -2651,7 +2688,7 @@ int tmnn_forward_for_training(tmnn_trainer *tr, const float *input, float *outpu
   if (!input || !output) return fail(TMNN_ERR_INVALID_ARGUMENT, "input/output is null");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   const int bn = std::min(n, tr->d.batch_size);
-  int rc = ensure_batch(tr, bn, sorts(tr, bn));
+  int rc = ensure_batch(tr, bn, sorts(tr, bn, kSortForward));
   if (rc != TMNN_OK) return rc;
   hipStream_t st = tr->ctx->stream;
   const size_t D = tr->d.spatial_dims, M = tr->d.num_outputs;
@@ -2660,7 +2697,8 @@ int tmnn_forward_for_training(tmnn_trainer *tr, const float *input, float *outpu
   if ((rc = stage_in(tr, input, tr->in_pos, bn * D * sizeof(float))) != TMNN_OK) return rc;
   const float *pos = nullptr, *unused = nullptr;
   const uint32_t *perm = nullptr;
-  rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, bn, &pos, &unused, &perm);
+  rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, bn, &pos, &unused, &perm,
+                  sorts(tr, bn, kSortForward));
   if (rc != TMNN_OK) return rc;
   FieldArgs a = base_args(tr);
   a.mode = kModeForward;
@@ -2691,7 +2729,7 @@ int tmnn_backward_accumulate(tmnn_trainer *tr, const float *input, const float *
   if (!input || !d_output) return fail(TMNN_ERR_INVALID_ARGUMENT, "input/d_output is null");
   TMNN_HIP_TRY(hipSetDevice(tr->ctx->device));
   const int bn = std::min(n, tr->d.batch_size);
-  int rc = ensure_batch(tr, bn, sorts(tr, bn));
+  int rc = ensure_batch(tr, bn, sorts(tr, bn, kSortHostPass));
   if (rc != TMNN_OK) return rc;
   hipStream_t st = tr->ctx->stream;
   StageLease lease(tr);
@@ -3076,7 +3114,8 @@ int tmnn_debug_encode_tiles(tmnn_trainer *tr, const float *positions, int32_t n,
   const float *pos = tr->in_pos.as<float>(), *unused = nullptr;
   const uint32_t *perm = nullptr;
   if (sorted) {
-    rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, n, &pos, &unused, &perm, false, true);
+    rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, n, &pos, &unused, &perm,
+                    tr->d.morton_sort && n > 1, false);
     if (rc != TMNN_OK) return rc;
   }
   float *pos_out = perm ? tr->s_pos.as<float>() : nullptr;
@@ -3119,8 +3158,8 @@ int tmnn_debug_hash_rates(tmnn_trainer *tr, const float *d_positions, int32_t n,
   if (rc != TMNN_OK) return rc;
   const float *pos = d_positions, *unused = nullptr;
   const uint32_t *perm = nullptr;
-  if (sorted && (rc = sort_batch(tr, d_positions, nullptr, 0, n, &pos, &unused, &perm, true, true)) !=
-                    TMNN_OK)
+  if (sorted && (rc = sort_batch(tr, d_positions, nullptr, 0, n, &pos, &unused, &perm,
+                                 tr->d.morton_sort && n > 1)) != TMNN_OK)
     return rc;
   TMNN_HIP_TRY(tr->dbg_a.ensure(static_cast<size_t>(tr->hash_count) * sizeof(int32_t)));
   TMNN_HIP_TRY(tr->dbg_b.ensure(tr->hash_entries));
@@ -3310,7 +3349,8 @@ int tmnn_debug_morton_sort(tmnn_trainer *tr, const float *positions, int32_t n, 
   TMNN_HIP_TRY(hipStreamSynchronize(st));
   const float *sp = nullptr, *stg = nullptr;
   const uint32_t *p = nullptr;
-  rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, n, &sp, &stg, &p, true, true);
+  rc = sort_batch(tr, tr->in_pos.as<float>(), nullptr, 0, n, &sp, &stg, &p,
+                  tr->d.morton_sort && n > 1);
   if (rc != TMNN_OK) return rc;
   if (!p && n == 1) {
     perm[0] = 0u;  // a single point is its own order
