@@ -100,3 +100,37 @@ def test_gradients_match_the_split_path(dims, feats, log2t, levels, n):
         assert np.count_nonzero(mb) > mb.size // 20
         assert np.abs(ma - mb).max() <= 16 * 0.1 / 65536 + 1e-6 * np.abs(mb).max()
         assert np.mean(ma != mb) <= 0.01
+
+
+def test_a_failed_step_leaves_no_visit_flags():
+    """A step that cannot allocate its activations (2^25 points times 8 layers of
+    512: 550 GB) fails after its visit pass was enqueued: the error is reported
+    once, and the next step moves the moments of its own corners only."""
+    torch = pytest.importorskip("torch")
+    from tiny_metal_nn._lib import TmnnError
+    n, log2t, levels = 1 << 17, 19, 2
+    big = 1 << 25
+    assert big * 512 * 8 * 4 > torch.cuda.get_device_properties(0).total_memory
+    print("failed step with a visit pass", flush=True)
+    rng = np.random.default_rng(9)
+    enc = dict(n_levels=levels, n_features_per_level=2, log2_hashmap_size=log2t,
+               base_resolution=64.0, per_level_scale=2.0)
+    with make_trainer(3, 1, enc, dict(n_neurons=512, n_hidden_layers=8), batch=big,
+                      hash_range=0.5) as tr:
+        tr.import_optimizer_state(_moments(tr, 1.0))
+        x = torch.rand(big, 3, device="cuda")
+        y = torch.zeros(big, 1, device="cuda")
+        torch.cuda.synchronize()
+        with pytest.raises(TmnnError, match="out of memory"):
+            tr.training_step_device(x.data_ptr(), y.data_ptr(), big)
+        assert tr.step() == 10
+        del x, y
+        pos = rng.random((n, 3), dtype=np.float32) * np.float32(0.25)
+        tr.training_step(pos, np.zeros((n, 1), np.float32))
+        want = np.zeros((levels, 1 << log2t), bool)
+        _, idx, _ = tr.debug_encode(pos, with_corners=True)
+        for lv in range(levels):
+            want[lv, idx[:, lv].ravel()] = True
+        assert 0.01 < want.mean() < 0.9
+        moved = (_m_of(tr) != 1.0).reshape(levels, 1 << log2t, 2).all(axis=2)
+        assert np.array_equal(moved, want)

@@ -237,7 +237,10 @@ struct DevBuf {
     }
     const size_t rounded = (want + 255) / 256 * 256;
     hipError_t e = hipMalloc(&ptr, rounded);
-    if (e == hipSuccess) bytes = rounded;
+    if (e == hipSuccess)
+      bytes = rounded;
+    else
+      (void)hipGetLastError();  // returned here; the next launch's check must not find it
     return e;
   }
   template <class T>
@@ -1645,11 +1648,22 @@ int sort_batch_overlapped(tmnn_trainer *tr, const float *d_pos, int n, bool stag
   TMNN_HIP_TRY(hipStreamWaitEvent(st, tr->ev_sorted[k], 0));
   if (visit) {
     TMNN_HIP_TRY(hipStreamWaitEvent(sd, tr->ev_flags_free, 0));
+    // the event follows whatever of the pass was enqueued, also when that failed
     const int rc = launch_visit(tr, d_pos, n, sd);
-    if (rc != TMNN_OK) return rc;
     TMNN_HIP_TRY(hipEventRecord(tr->ev_visited, sd));
     tr->visit_pending = true;
+    return rc;
   }
+  return TMNN_OK;
+}
+
+// The main stream waits for the visit pass of the step being enqueued, where
+// the side stream has one: before the finish kernel, and in a step that fails
+// (the pass reads the caller's positions and writes visit_bits and the flags).
+int visit_join(tmnn_trainer *tr) {
+  if (!tr->visit_pending) return TMNN_OK;
+  tr->visit_pending = false;
+  TMNN_HIP_TRY(hipStreamWaitEvent(tr->ctx->stream, tr->ev_visited, 0));
   return TMNN_OK;
 }
 
@@ -1662,6 +1676,28 @@ int sort_set_consumed(tmnn_trainer *tr) {
   tr->consumed_recorded[k] = true;
   tr->sort_parity = (k + 1) % tmnn_trainer::kSortSets;
   return TMNN_OK;
+}
+
+int zero_device(tmnn_trainer *tr, void *ptr, size_t bytes) {
+  if (bytes == 0) return TMNN_OK;
+  const size_t n16 = (bytes + 15) / 16;
+  const uint32_t blocks = static_cast<uint32_t>(
+      std::min<size_t>((n16 + 255) / 256, static_cast<size_t>(tr->ctx->cu_count) * 8));
+  hipLaunchKernelGGL(zero_bytes_kernel, dim3(std::max<uint32_t>(blocks, 1)), dim3(256), 0,
+                     tr->ctx->stream, static_cast<uint8_t *>(ptr), bytes);
+  TMNN_HIP_TRY(hipGetLastError());
+  return TMNN_OK;
+}
+
+// The flags that a step's visit pass stored, taken back: the step failed with
+// status rc before its backward, and the next step's Adam must not move their
+// entries.
+int visit_drop(tmnn_trainer *tr, int rc) {
+  const std::string why = g_last_error;
+  (void)visit_join(tr);
+  (void)zero_device(tr, tr->mask[tr->mask_cur].ptr, tr->hash_entries);
+  g_last_error = why;
+  return rc;
 }
 
 // Fused forward/backward over n device-resident points, gradients
@@ -1683,12 +1719,12 @@ int run_forward_backward(tmnn_trainer *tr, const float *d_pos, const float *d_tg
     // feature-tile plans read the batch through the permutation (no gather)
     rc = sort_batch_overlapped(tr, d_pos, n, overlap_sort > 1, visit, &perm);
   } else {
-    if (visit && (rc = launch_visit(tr, d_pos, n, tr->ctx->stream)) != TMNN_OK) return rc;
-    rc = sort_batch(tr, d_pos, d_tgt, tr->d.num_outputs, n, &pos, &tgt, &perm, order,
-                    !tr->train_plan.xmem);
+    if (visit) rc = launch_visit(tr, d_pos, n, tr->ctx->stream);
+    if (rc == TMNN_OK)
+      rc = sort_batch(tr, d_pos, d_tgt, tr->d.num_outputs, n, &pos, &tgt, &perm, order,
+                      !tr->train_plan.xmem);
   }
-  if (rc != TMNN_OK) return rc;
-  if ((rc = prof_mark(tr, 1)) != TMNN_OK) return rc;
+  if (rc != TMNN_OK || (rc = prof_mark(tr, 1)) != TMNN_OK) return visit ? visit_drop(tr, rc) : rc;
   FieldArgs a = base_args(tr);
   a.mode = external_grad ? kModeTrainExtGrad : kModeTrainLoss;
   a.inv_n = 1.0f / static_cast<float>(n);
@@ -1716,7 +1752,7 @@ int run_forward_backward(tmnn_trainer *tr, const float *d_pos, const float *d_tg
     a.mask = visit ? nullptr : tr->mask[tr->mask_cur].as<uint8_t>();
   }
   const int blocks = launch_field(tr, tr->train_plan, a, n, 2, false, a.tgt_index, sorted_pos);
-  if (blocks < 0) return blocks;
+  if (blocks < 0) return visit ? visit_drop(tr, blocks) : blocks;
   if ((rc = prof_mark(tr, 3)) != TMNN_OK) return rc;
   if (!fused_scatter) {  // else the scatter phase is empty (no boundary event)
     if ((rc = launch_scatter(tr, indexed ? sorted_pos : pos, n, visit)) != TMNN_OK) return rc;
@@ -1868,17 +1904,6 @@ int launch_pos_grad(tmnn_trainer *tr, const PosGradArgs &g) {
   return TMNN_OK;
 }
 
-int zero_device(tmnn_trainer *tr, void *ptr, size_t bytes) {
-  if (bytes == 0) return TMNN_OK;
-  const size_t n16 = (bytes + 15) / 16;
-  const uint32_t blocks = static_cast<uint32_t>(
-      std::min<size_t>((n16 + 255) / 256, static_cast<size_t>(tr->ctx->cu_count) * 8));
-  hipLaunchKernelGGL(zero_bytes_kernel, dim3(std::max<uint32_t>(blocks, 1)), dim3(256), 0,
-                     tr->ctx->stream, static_cast<uint8_t *>(ptr), bytes);
-  TMNN_HIP_TRY(hipGetLastError());
-  return TMNN_OK;
-}
-
 // Releases the event set claimed for a step that failed before its last
 // event was recorded (prof_collect would otherwise read unrecorded events).
 void prof_abort(tmnn_trainer *tr) {
@@ -1966,15 +1991,13 @@ int train_step_device(tmnn_trainer *tr, const float *d_pos, const float *d_tgt, 
   tr->input_ready = input_ready;
   const int blocks = run_forward_backward(tr, d_pos, d_tgt, n, false, loss, false, overlap_sort);
   tr->input_ready = nullptr;
-  if (blocks < 0) {
+  // the finish kernel, or whatever follows a step that failed, comes after the visit pass
+  rc = visit_join(tr);
+  if (blocks < 0 || rc != TMNN_OK) {
     tr->num_this_step = false;
     prof_abort(tr);
     if (overlapped) (void)sort_set_consumed(tr);
-    return blocks;
-  }
-  if (tr->visit_pending) {
-    tr->visit_pending = false;
-    TMNN_HIP_TRY(hipStreamWaitEvent(tr->ctx->stream, tr->ev_visited, 0));
+    return blocks < 0 ? blocks : rc;
   }
   // dW reduction, loss and Adam in one kernel (the reduce phase is empty: no
   // boundary event)
