@@ -134,3 +134,36 @@ def test_a_failed_step_leaves_no_visit_flags():
         assert 0.01 < want.mean() < 0.9
         moved = (_m_of(tr) != 1.0).reshape(levels, 1 << log2t, 2).all(axis=2)
         assert np.array_equal(moved, want)
+
+
+@pytest.mark.parametrize("dims,log2t,n", [(3, 19, 131072), (4, 16, 131072)])
+def test_steps_enqueued_back_to_back(dims, log2t, n):
+    """Steps without a wait between them, an allocation-free one (whose visit
+    pass runs on the main stream) among them, over batches in different
+    places: weights and moments equal, to the bit, those of a trainer that is
+    waited for after every step. Needs a step's pass after the last finish
+    kernel cleared the flags, and its finish kernel after its pass."""
+    torch = pytest.importorskip("torch")
+    print(f"back to back {dims}D T2^{log2t}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(dims)
+    batches = []
+    for i in range(6):
+        x = torch.rand(n, dims, device="cuda", generator=g)
+        x[:, 0] = (x[:, 0] + i) / 6
+        batches.append((x.contiguous(), torch.rand(n, 2, device="cuda", generator=g)))
+    torch.cuda.synchronize()
+    enc = dict(n_levels=8, n_features_per_level=2, log2_hashmap_size=log2t, base_resolution=16.0,
+               per_level_scale=1.5)
+    got = []
+    for wait in (True, False):
+        with make_trainer(dims, 2, enc, dict(n_neurons=64, n_hidden_layers=2), loss="L2",
+                          batch=n, hash_range=0.5) as tr:
+            tr.import_optimizer_state(_moments(tr, 1.0))
+            for i, (x, y) in enumerate(batches):
+                step = tr.training_step_device_noalloc if i == 3 else tr.training_step_device
+                step(x.data_ptr(), y.data_ptr(), n)
+                if wait:
+                    tr.synchronize()
+            got.append((*tr.get_weights(), _m_of(tr).copy()))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
