@@ -102,6 +102,33 @@ def test_gradients_match_the_split_path(dims, feats, log2t, levels, n):
         assert np.mean(ma != mb) <= 0.01
 
 
+def test_trainers_of_different_table_sizes():
+    """A trainer whose visit pass takes 128 KB of LDS steps after one with a
+    smaller table was created (both launch the same kernel), and the smaller
+    one after it."""
+    rng = np.random.default_rng(4)
+    n = 1 << 18
+    pos, tgt = rng.random((n, 3), dtype=np.float32), rng.random((n, 1), dtype=np.float32)
+    net = dict(n_neurons=32, n_hidden_layers=1)
+
+    def enc(log2t):
+        return dict(n_levels=2, n_features_per_level=2, log2_hashmap_size=log2t,
+                    base_resolution=256.0, per_level_scale=2.0)
+
+    print("two table sizes", flush=True)
+    with make_trainer(3, 1, enc(20), net, batch=n) as large, \
+            make_trainer(3, 1, enc(10), net, batch=n) as small:
+        for tr, log2t in ((large, 20), (small, 10), (large, 20)):
+            tr.import_optimizer_state(_moments(tr, 1.0))
+            tr.training_step(pos, tgt)
+            want = np.zeros((2, 1 << log2t), bool)
+            _, idx, _ = tr.debug_encode(pos, with_corners=True)
+            for lv in range(2):
+                want[lv, idx[:, lv].ravel()] = True
+            moved = (_m_of(tr) != 1.0).reshape(2, 1 << log2t, 2).all(axis=2)
+            assert np.array_equal(moved, want)
+
+
 def test_a_failed_step_leaves_no_visit_flags():
     """A step that cannot allocate its activations (2^25 points times 8 layers of
     512: 550 GB) fails after its visit pass was enqueued: the error is reported

@@ -2368,11 +2368,12 @@ int tmnn_trainer_create(tmnn_context *ctx, const tmnn_model_desc *desc, tmnn_tra
   if (visit_pass(tr.get(), desc->batch_size)) {
     const VisitShape vs = visit_shape(tr.get(), desc->batch_size);
     TMNN_HIP_TRY(tr->visit_bits.ensure(static_cast<size_t>(vs.shares) * (tr->hash_entries / 8u)));
-    const int log2R = std::min<int>(desc->log2_hashmap_size, kVisitLog2Range);
+    // the attribute is the function's, which trainers of every table size
+    // share: the largest range, not this trainer's
     TMNN_HIP_TRY(hipFuncSetAttribute(
-        reinterpret_cast<const void *>(
-            visit_kernel_of(desc->spatial_dims, desc->log2_hashmap_size > log2R)),
-        hipFuncAttributeMaxDynamicSharedMemorySize, 1 << (log2R - 3)));
+        reinterpret_cast<const void *>(visit_kernel_of(
+            desc->spatial_dims, desc->log2_hashmap_size > static_cast<int>(kVisitLog2Range))),
+        hipFuncAttributeMaxDynamicSharedMemorySize, 1 << (kVisitLog2Range - 3)));
   }
   if ((rc = plan_kernel(tr.get(), tr->d.precision == TMNN_PRECISION_FP16, false,
                         tr->fwd_plan)) != TMNN_OK)
