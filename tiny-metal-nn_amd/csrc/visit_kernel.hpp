@@ -41,7 +41,9 @@ struct VisitArgs {
 typedef __attribute__((address_space(3))) uint32_t visit_word;
 
 __device__ __forceinline__ visit_word *visit_word_at(uint32_t byte) {
-  // the bits are the kernel's only LDS: they start at address 0
+  // the bits are the kernel's only LDS: they start at address 0 (checked when
+  // a trainer is created; through the array's own address the kernels take 5%
+  // more instructions)
   return reinterpret_cast<visit_word *>(byte);
 }
 
