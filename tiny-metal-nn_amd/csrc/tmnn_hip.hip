@@ -2368,12 +2368,17 @@ int tmnn_trainer_create(tmnn_context *ctx, const tmnn_model_desc *desc, tmnn_tra
   if (visit_pass(tr.get(), desc->batch_size)) {
     const VisitShape vs = visit_shape(tr.get(), desc->batch_size);
     TMNN_HIP_TRY(tr->visit_bits.ensure(static_cast<size_t>(vs.shares) * (tr->hash_entries / 8u)));
+    const void *fn = reinterpret_cast<const void *>(visit_kernel_of(
+        desc->spatial_dims, desc->log2_hashmap_size > static_cast<int>(kVisitLog2Range)));
+    // visit_word_at's addresses count from the start of the block's LDS
+    hipFuncAttributes attr{};
+    TMNN_HIP_TRY(hipFuncGetAttributes(&attr, fn));
+    if (attr.sharedSizeBytes != 0)
+      return fail(TMNN_ERR_RUNTIME, "visit_kernel has static LDS before its bits");
     // the attribute is the function's, which trainers of every table size
     // share: the largest range, not this trainer's
-    TMNN_HIP_TRY(hipFuncSetAttribute(
-        reinterpret_cast<const void *>(visit_kernel_of(
-            desc->spatial_dims, desc->log2_hashmap_size > static_cast<int>(kVisitLog2Range))),
-        hipFuncAttributeMaxDynamicSharedMemorySize, 1 << (kVisitLog2Range - 3)));
+    TMNN_HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     1 << (kVisitLog2Range - 3)));
   }
   if ((rc = plan_kernel(tr.get(), tr->d.precision == TMNN_PRECISION_FP16, false,
                         tr->fwd_plan)) != TMNN_OK)
