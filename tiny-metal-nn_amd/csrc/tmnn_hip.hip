@@ -2178,10 +2178,12 @@ int tmnn_context_create(int32_t device, tmnn_context **out) {
   TMNN_HIP_TRY(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
   {  // without pinned memory the host-pointer calls copy through hipMemcpyAsync
     void *p = nullptr;
-    if (hipHostMalloc(&p, kStageTotal, hipHostMallocDefault) == hipSuccess)
+    if (hipHostMalloc(&p, kStageTotal, hipHostMallocDefault) == hipSuccess) {
       ctx->stage = static_cast<unsigned char *>(p);
-    else
+      std::memset(p, 0, kStageTotal);  // maps its pages here, not in the first calls
+    } else {
       (void)hipGetLastError();
+    }
   }
   {
     // This device's copy of the step scratch, with the device current, and
