@@ -39,14 +39,16 @@ def test_outputs_and_gradients_match_oracle(oracle, width, layers, m, n):
         assert rel_tensor(gm, ogm) <= 1e-5
 
 
-@pytest.mark.parametrize("width,n", [(128, 70001), (256, 40000), (96, 3000)])
-def test_forward_error_against_64_bits(width, n):
+@pytest.mark.parametrize("width,n,bound", [
+    (128, 70001, 2.2e-7), (256, 40000, 3.3e-7), (96, 3000, 1.8e-7)])
+def test_forward_error_against_64_bits(width, n, bound):
     """Both tile widths (128 columns from four blocks a CU on): the 2-norm error
     against 64 bits stays below that of the fp32 MFMA tiles at the same shape
     and inputs (2.6e-7, 4.3e-7, 2.1e-7; the split products 1.8e-7, 2.5e-7,
-    1.5e-7). Bound: per layer K / 32 roundings of the accumulator at 2^-24, a
-    random walk of sqrt(8) * 6e-8 = 1.7e-7 at K = 256 and once more for bias
-    and output, over three layers in quadrature below 4e-7."""
+    1.5e-7). Bounds halfway between the two, so that neither the fp32 tiles nor
+    split products as inexact as them pass; K / 32 roundings of the accumulator
+    at 2^-24, a random walk of sqrt(8) * 6e-8 = 1.7e-7 a layer at K = 256, lie
+    below."""
     print(f"split products error w{width} n{n}", flush=True)
     rng = np.random.default_rng(width)
     with make_trainer(3, 4, ENC, dict(n_neurons=width, n_hidden_layers=3), hash_range=0.5,
@@ -61,7 +63,79 @@ def test_forward_error_against_64_bits(width, n):
             at += a * b + b
             if i < 3:
                 x = np.maximum(x, 0)
-        assert np.linalg.norm(out - x) <= 4e-7 * np.linalg.norm(x)
+        assert np.linalg.norm(out - x) <= bound * np.linalg.norm(x)
+
+
+# (width, points): 128-column tiles in the delta, dx and (256 wide) weight-
+# gradient products, over many chunks of the batch; 64-column ones and few
+# chunks. Bounds of the split products' dW1, db1 and, through dx, the table,
+# halfway between their errors (3.5e-7, 4.4e-7, 3.5e-6; 2.2e-7, 2.2e-7, 2.6e-6;
+# 1.7e-7, 1.9e-7, 3.7e-6) and the fp32 MFMA tiles' (9.8e-7, 8.9e-7, 5.2e-6;
+# 5.7e-7, 4.6e-7, 3.8e-6; 4.4e-7, 4.4e-7, 5.2e-6)
+@pytest.mark.parametrize("width,n,dw1,db1,table", [
+    (256, 66001, 6.5e-7, 6.5e-7, 4.3e-6), (128, 70001, 4e-7, 3.4e-7, 3.2e-6),
+    (256, 3001, 3e-7, 3.1e-7, 4.4e-6)])
+def test_gradient_error_against_64_bits(width, n, dw1, db1, table):
+    """Weight, bias and table gradients of a step's backward against 64 bits on
+    the same features, with pre-activations kept away from 0 by the biases (no
+    ReLU mask that a rounding decides). The first and last layers' products are
+    fp32 ones in both (2.3e-7 to 1.2e-6): below twice the largest. Of the
+    table's error most is the fixed point's truncation, which an ulp of d can
+    move."""
+    torch = pytest.importorskip("torch")
+    print(f"split gradients error w{width} n{n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(width + n)
+    enc = dict(n_levels=16, n_features_per_level=2, log2_hashmap_size=12, base_resolution=8.0,
+               per_level_scale=1.3)
+    sizes = [32, width, width, 4]
+    rng = np.random.default_rng(n)
+    with make_trainer(3, 4, enc, dict(n_neurons=width, n_hidden_layers=2), hash_range=0.5,
+                      batch=n) as tr:
+        hw, mw = (w.copy() for w in tr.get_weights())
+        at, spans = 0, []
+        for i, (a, b) in enumerate(zip(sizes, sizes[1:])):
+            spans.append((at, at + a * b, at + a * b + b))
+            if i < 2:
+                mw[spans[-1][1]:spans[-1][2]] = np.where(np.arange(b) % 2, 4.0, -4.0) * (1 + 7 * i)
+            at = spans[-1][2]
+        tr.set_initial_weights(hw, mw)
+        pos = rng.random((n, 3), dtype=np.float32)
+        dout = rng.normal(0, 1.0, (n, 4)).astype(np.float32)
+        feats, idx, wts = tr.debug_encode(pos, with_corners=True)
+        tr.zero_gradients()
+        tr.backward_accumulate(pos, dout)
+        gh, gm = tr.debug_gradients()
+        w = [torch.from_numpy(mw[p:q].reshape(a, b)).cuda().double()
+             for (p, q, _), a, b in zip(spans, sizes, sizes[1:])]
+        bias = [torch.from_numpy(mw[q:r]).cuda().double() for _, q, r in spans]
+        acts = [torch.from_numpy(feats).cuda().double()]
+        for i in range(2):
+            z = acts[-1] @ w[i] + bias[i]
+            assert float(z.abs().min()) > 1e-4
+            acts.append(z.relu())
+        d, errors = torch.from_numpy(dout).cuda().double(), {}
+        for i in (2, 1, 0):
+            p, q, r = spans[i]
+            for key, lo, hi, want in ((f"dW{i}", p, q, (acts[i].T @ d).flatten()),
+                                      (f"db{i}", q, r, d.sum(0))):
+                got = torch.from_numpy(gm[lo:hi]).cuda().double()
+                errors[key] = float((got - want).norm() / want.norm())
+            d = d @ w[i].T.contiguous()
+            if i:
+                d *= acts[i] > 0
+        # the table's fixed point: every contribution times 65536, truncated
+        want = torch.zeros(16, 1 << 12, 2, dtype=torch.float64, device="cuda")
+        ci, cw = torch.from_numpy(idx.astype(np.int64)).cuda(), torch.from_numpy(wts).cuda().double()
+        for lv in range(16):
+            for c in range(8):
+                want[lv].index_add_(0, ci[:, lv, c], torch.trunc(
+                    d[:, 2 * lv:2 * lv + 2] * cw[:, lv, c, None] * 65536))
+        got = torch.from_numpy(gh.astype(np.float64)).cuda().view_as(want)
+        errors["table"] = float((got - want).norm() / want.norm())
+        print(" ".join(f"{k} {v:.2e}" for k, v in errors.items()), flush=True)
+        bounds = {"dW1": dw1, "db1": db1, "table": table}
+        for key, error in errors.items():
+            assert error <= bounds.get(key, 2.4e-6), (key, error)
 
 
 def _forward64(mw, sizes, x):

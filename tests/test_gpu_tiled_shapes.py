@@ -88,7 +88,7 @@ def test_tiled_plan_and_inference(oracle, name):
             ref = oracle.forward(omodel(oracle, tr), hw, mw, pos)
             tol = 1e-5 * (np.abs(ref) + np.sqrt((ref.astype(np.float64) ** 2).mean()))
             assert np.all(np.abs(out - ref) <= tol), (n, float(np.abs(out - ref).max()))
-        # forward_for_training: caller's point order through the Morton sort
+        # forward_for_training: the caller's point order (batches this small in input order)
         a = tr.forward_for_training(pos)
         tol = 1e-5 * (np.abs(ref) + np.sqrt((ref.astype(np.float64) ** 2).mean()))
         assert np.all(np.abs(a - ref) <= tol)

@@ -31,6 +31,9 @@ CASES = {
     "3d_fp32": ("3d_f2", "fp32", "auto", (20000, 777)),
     "3d_f4_fp16": ("3d_f4", "fp16", "auto", (9000, 4100)),
     "2d_tiled": ("2d_f2", "fp16", "Tiled", (6000, 3001)),
+    # above the size from which every 3D batch is sorted and takes the visit pass
+    "3d_sorted": ("3d_f2", "fp32", "auto", (1 << 17, 131201)),
+    "4d_sorted": ("4d_f2", "fp32", "auto", (20000, 9001)),
 }
 
 
@@ -72,20 +75,25 @@ def test_noalloc_step_matches_device_step(case):
                  f"{np.array_equal(mn, mr) and np.array_equal(hn, hr)}")
 
 
-def test_noalloc_alternating_with_regular_steps_on_one_trainer():
+# batches all unsorted (2D, a training kernel with its own hash-grid backward);
+# sorted and unsorted ones in turn; a separate hash-grid backward, all sorted
+@pytest.mark.parametrize("geom,sizes", [
+    ("2d_f2", (20000, 8192, 20000, 3001, 12345, 20000)),
+    ("2d_f2", (70001, 40000, 8192, 70001, 40000, 12345, 70001)),
+    ("3d_f4", (20000, 8192, 20000, 3001, 12345, 20000))])
+def test_noalloc_alternating_with_regular_steps_on_one_trainer(geom, sizes):
     """Regular, allocation-free, regular, allocation-free steps on one trainer
     (the regular steps sort on the side stream into their buffer sets, the
     allocation-free ones on the main stream into the scratch, lending and
     restoring the trainer's batch buffers) against a trainer that takes only
     regular steps: losses and weights bit-identical after every step."""
     torch = pytest.importorskip("torch")
-    d, enc, net, m_out = GEOMS["2d_f2"]
-    _say("noalloc alternating")
+    d, enc, net, m_out = GEOMS[geom]
+    _say(f"noalloc alternating {geom} {sizes}")
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(21)
-    sizes = (20000, 8192, 20000, 3001, 12345, 20000)
-    with make_trainer(d, m_out, enc, net, precision="fp16", batch=20000, hash_range=0.1) as ref, \
-            make_trainer(d, m_out, enc, net, precision="fp16", batch=20000, hash_range=0.1) as tr:
+    with make_trainer(d, m_out, enc, net, precision="fp16", batch=max(sizes), hash_range=0.1) as ref, \
+            make_trainer(d, m_out, enc, net, precision="fp16", batch=max(sizes), hash_range=0.1) as tr:
         for i, n in enumerate(sizes):
             x = torch.rand(n, d, device=dev, generator=g)
             y = torch.rand(n, m_out, device=dev, generator=g)
