@@ -6,7 +6,8 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from test_gpu_parity import GEOMS, away_from_relu_kinks, make_trainer, omodel, rel_tensor
+from test_gpu_parity import (GEOMS, _compact_2d, away_from_relu_kinks, make_trainer, omodel,
+                             rel_tensor)
 
 pytestmark = pytest.mark.gpu
 
@@ -14,7 +15,7 @@ pytestmark = pytest.mark.gpu
 # the smallest sorted batch of the plans whose separate hash-grid backward
 # merges runs of lanes on one entry, for host-pointer and device-pointer steps
 @pytest.mark.parametrize("dims,feats,host,n", [
-    (3, 1, True, 4097), (3, 1, False, 1025), (2, 1, True, 2049), (2, 1, False, 33),
+    (3, 1, True, 4097), (3, 1, False, 1025), (2, 1, True, 1025), (2, 1, False, 33),
     (3, 4, True, 33), (3, 4, False, 33), (2, 4, True, 33), (4, 2, True, 8193), (4, 2, False, 8193)])
 def test_sorted_steps_do_not_depend_on_the_row_order(dims, feats, host, n):
     """The sort is stable, so a batch and its sorted copy take the same order: the
@@ -74,3 +75,22 @@ def test_sorted_backward_matches_oracle(oracle, name, n):
         assert rel_tensor(gm, ogm) <= 1e-5
         diff = np.abs(gh.astype(np.int64) - ogh.astype(np.int64))
         assert (diff == 0).mean() > 0.99 and diff.max() <= 16, int(diff.max())
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
+def test_one_block_sort(oracle, dims):
+    """Batches up to 8192 points are sorted by one kernel: codes and a stable
+    order at the sizes around its waves' and instances' shares, with repeated
+    points, points outside the domain and (4D, whose codes repeat) long ties."""
+    rng = np.random.default_rng(dims)
+    enc = dict(n_levels=2, n_features_per_level=2, log2_hashmap_size=10, base_resolution=4.0,
+               per_level_scale=2.0)
+    with make_trainer(dims, 1, enc, dict(n_neurons=32, n_hidden_layers=1), batch=8193) as tr:
+        for n in (2, 63, 65, 256, 257, 511, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, 6000, 8191, 8192, 8193):
+            print(f"one-block sort {dims}D n{n}", flush=True)
+            pos = rng.random((n, dims), dtype=np.float32) * np.float32(2.4) - np.float32(1.2)
+            pos[n // 2:] = pos[rng.integers(0, n - n // 2, n - n // 2)]
+            codes, perm = tr.debug_morton_sort(pos)
+            want = oracle.morton_codes(pos, dims)
+            assert np.array_equal(codes, _compact_2d(want) if dims == 2 else want)
+            assert np.array_equal(perm, np.argsort(codes, kind="stable"))

@@ -20,7 +20,8 @@
 //             chunk locally in LDS and writes it out digit run by digit run,
 //             so consecutive lanes store consecutive addresses; the 2D MSD
 //             pass also writes each digit's output start for the buckets.
-// Ties keep input order (stable), so the sorted order is deterministic.
+// Ties keep input order (stable), so the sorted order is deterministic. Batches
+// up to kSmallSortKeys points take one kernel instead (small_sort_kernel).
 #include "sort.hpp"
 
 #include <algorithm>
@@ -215,7 +216,7 @@ __device__ __forceinline__ void clear_counts(ChunkLds<RB, KPT> &L) {
 // Every wave ranks its keys, 64 per round in input order, against its own
 // counters (no barriers): piw = keys of the same digit before it in the wave.
 template <int RB, int KPT>
-__device__ __forceinline__ void rank_in_waves(ChunkLds<RB, KPT> &L, const uint32_t (&key)[KPT],
+__device__ __forceinline__ void rank_in_waves(uint16_t (*wcnt)[1 << RB], const uint32_t (&key)[KPT],
                                               int nblk, int shift, uint32_t (&piw)[KPT]) {
   constexpr int kBins = 1 << RB;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -234,9 +235,9 @@ __device__ __forceinline__ void rank_in_waves(ChunkLds<RB, KPT> &L, const uint32
     const uint32_t rank = static_cast<uint32_t>(__popcll(peers & lt_mask));
     // every lane reads the wave's running count before the leader advances
     // it (the LDS operations of one wave complete in program order)
-    const uint32_t c = valid ? L.wcnt[wave][d] : 0u;
+    const uint32_t c = valid ? wcnt[wave][d] : 0u;
     piw[r] = c + rank;
-    if (valid && rank == 0u) L.wcnt[wave][d] = static_cast<uint16_t>(c + __popcll(peers));
+    if (valid && rank == 0u) wcnt[wave][d] = static_cast<uint16_t>(c + __popcll(peers));
   }
 }
 
@@ -335,7 +336,7 @@ __global__ void __launch_bounds__(kSortThreads)
     }
     key[r] = valid ? key[r] : 0u;
   }
-  rank_in_waves(L, key, nblk, shift, piw);
+  rank_in_waves<RB, KPT>(L.wcnt, key, nblk, shift, piw);
   __syncthreads();
 
   // the chunk's count of each owned digit, the run's start in the chunk and
@@ -421,7 +422,7 @@ __global__ void __launch_bounds__(kSortThreads)
       key[r] = valid ? keys_in[gi] : 0u;
       val[r] = valid ? vals_in[gi] : 0u;
     }
-    rank_in_waves(L, key, nblk, 0, piw);
+    rank_in_waves<RB, KPT>(L.wcnt, key, nblk, 0, piw);
     __syncthreads();
     uint32_t cnt[BPT], sc = 0;
     wave_offsets(L, cnt);
@@ -446,6 +447,92 @@ __global__ void __launch_bounds__(kSortThreads)
     __syncthreads();
     write_chunk(L, nblk, 0, keys_out, vals_out);
     __syncthreads();  // L is reused by the next chunk
+  }
+}
+
+// A batch of at most 1024 KPT points, sorted in one block: its codes and rows
+// stay in registers and LDS over the LSD passes, 8 bits each. The three kernels
+// per pass and the second stream's events took 67 us of a synchronous step of
+// 4096 3D points (157 us against 90 unsorted); with this kernel on the step's
+// own stream the step takes 110. Bound by the wave ballots of the ranking on
+// one CU: 7 to 9 us up to 1024 points, 12 up to 2048, 19 at 4096, 33 at 8192,
+// where the many-block passes take over.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / 64;
+static_assert(kSmallSortKeys == kSmallThreads * 8, "largest instance");
+
+template <int KPT>
+__global__ void __launch_bounds__(kSmallThreads)
+    small_sort_kernel(const float *pos, int dims, int n, int passes, uint32_t *keys_out,
+                      uint32_t *vals_out) {
+  constexpr int RB = 8, kBins = 1 << RB, kScanWaves = kBins / 64;
+  __shared__ uint32_t lkeys[kSmallThreads * KPT];
+  __shared__ uint16_t lvals[kSmallThreads * KPT];
+  __shared__ uint16_t wcnt[kSmallWaves][kBins];  // per-wave counts, then places (< the batch)
+  __shared__ uint32_t wsum[kScanWaves];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  uint32_t key[KPT], val[KPT], piw[KPT];
+  size_t gi[KPT];
+#pragma unroll
+  for (int r = 0; r < KPT; ++r) {
+    const int i = chunk_index<KPT>(r);
+    gi[r] = static_cast<size_t>(i < n ? i : 0);
+    val[r] = static_cast<uint32_t>(i);
+  }
+  load_keys<true, KPT>(nullptr, pos, dims, gi, key);
+  for (int pass = 0; pass < passes; ++pass) {  // uniform
+    const int shift = RB * pass;
+    for (int i = t; i < kSmallWaves * kBins / 2; i += kSmallThreads)
+      reinterpret_cast<uint32_t *>(&wcnt[0][0])[i] = 0u;
+    __syncthreads();
+    rank_in_waves<RB, KPT>(wcnt, key, n, shift, piw);
+    __syncthreads();
+    // thread t < 256 turns digit t's counts into each wave's first place
+    uint32_t total = 0;
+    if (t < kBins) {
+#pragma unroll
+      for (int w = 0; w < kSmallWaves; ++w) total += wcnt[w][t];
+    }
+    const uint32_t inc = wave_incl_scan(total, lane);
+    if (wave < kScanWaves && lane == 63) wsum[wave] = inc;
+    __syncthreads();
+    if (t < kBins) {
+      uint32_t place = inc - total;
+#pragma unroll
+      for (int k = 0; k < kScanWaves; ++k) place += k < wave ? wsum[k] : 0u;
+#pragma unroll
+      for (int w = 0; w < kSmallWaves; ++w) {
+        const uint32_t c = wcnt[w][t];
+        wcnt[w][t] = static_cast<uint16_t>(place);
+        place += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) {
+      if (chunk_index<KPT>(r) < n) {
+        const uint32_t p = wcnt[wave][(key[r] >> shift) & (kBins - 1)] + piw[r];
+        lkeys[p] = key[r];
+        lvals[p] = static_cast<uint16_t>(val[r]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < KPT; ++r) {
+      const int i = chunk_index<KPT>(r);
+      if (i < n) {
+        key[r] = lkeys[i];
+        val[r] = lvals[i];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < KPT; ++r) {
+    const int i = chunk_index<KPT>(r);
+    if (i < n) {
+      keys_out[i] = key[r];
+      vals_out[i] = val[r];
+    }
   }
 }
 
@@ -520,6 +607,17 @@ hipError_t morton_sort_batch(void *tmp, size_t tmp_bytes, const float *pos, int 
   // 2D codes interleave x and y only (the lifted z = 0 bits are all zero,
   // which leaves the order unchanged): 20 bits; 3D 30 bits; 4D 32 bits.
   const int end_bit = dims == 2 ? 20 : (dims == 3 ? 30 : 32);
+  if (n <= kSmallSortKeys) {
+    const auto fn = n <= kSmallThreads       ? small_sort_kernel<1>
+                    : n <= kSmallThreads * 2 ? small_sort_kernel<2>
+                    : n <= kSmallThreads * 4 ? small_sort_kernel<4>
+                                             : small_sort_kernel<8>;
+    hipLaunchKernelGGL(fn, dim3(1), dim3(kSmallThreads), 0, stream, pos, dims, n,
+                       (end_bit + 7) / 8, keys0, vals0);
+    *keys_sorted = keys0;
+    *vals_sorted = vals0;
+    return hipGetLastError();
+  }
   const size_t bins = size_t(1) << digit_bits(end_bit);
   const int blocks = sort_blocks(n, digit_bits(end_bit) == 8 ? kKeysPerThread : kKeysPerThread2D);
   uint32_t *hist = static_cast<uint32_t *>(tmp);

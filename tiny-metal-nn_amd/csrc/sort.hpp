@@ -9,6 +9,9 @@
 
 namespace tmnn_hip {
 
+// Batches up to this size are sorted by one kernel.
+constexpr int kSmallSortKeys = 8192;
+
 // Scratch bytes morton_sort_batch needs for n points.
 hipError_t morton_sort_temp_bytes(int n, size_t *bytes);
 

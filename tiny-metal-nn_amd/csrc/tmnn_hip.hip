@@ -1329,9 +1329,8 @@ enum SortPass {
 };
 
 // Whether a batch is put in Morton order at all: where its order saves more
-// gather and scatter time than the sort's kernels (twelve in 3D and 4D, four
-// in 2D, on a second stream in the fused device step) and their events cost.
-// Results differ by the order of their fp32 sums only.
+// gather and scatter time than the sort and its events cost. Results differ by
+// the order of their fp32 sums only.
 //
 // Forward passes, and training kernels that run the hash-grid backward
 // themselves (tile_scatter: no merging across lanes, so the order only moves
@@ -1345,16 +1344,17 @@ enum SortPass {
 //
 // The separate hash-grid backward merges the runs of lanes that share an entry
 // (scatter_kernel.hpp), which only a sorted batch has: without them clustered
-// points meet in the atomics (sorted / unsorted, us: 3D 8x4 T = 2^17 131071
-// points over 1/50 of the domain 1618 / 11803, 3D 8x2 32768 186 / 803, 2D 8x2
-// 8192 86 / 235, spread ones 3D 8x2 131071 387 / 599). It is left out only up
-// to the sizes where even that costs no more than the sort does, at worst
-// 0.95 over those spreads and gradients: host passes 16x2 T = 2^17: 3D 4096
-// points 157 / 89 spread, 173 / 181 clustered (8192: 196 / 273), 2D 2048
-// 152 / 100, 137 / 139 (4096: 154 / 185), 4D 8192 201 / 121, 524 / 479; device
-// steps 3D 1024 69 / 52, 79 / 76 (2048: 83 / 104), 4D 8192 106 / 92, 437 / 448,
-// none in 2D (512: 69 / 82). Four features (16x4) add by four 32-bit atomics
-// and lose in 2D and 3D at once (3D 1024: host 212 / 235, device 135 / 211).
+// points meet in the atomics (3D 8x4 T = 2^17 131071 points over 1/50 of the
+// domain 1618 / 11803, 3D 8x2 32768 points 186 / 803, 2D 107 / 550, 4D
+// 1034 / 1284, spread over all of it 3D 8x2 131071 points 387 / 599). There the
+// sort is left out up to the sizes where sorted / unsorted times, over those
+// spreads and gradients, pass 1 in the mean. 16x2 and 16x1, T = 2^17: host
+// passes 3D 4096 points 1.00 (110 / 90 spread, 123 / 181 clustered; 8192:
+// 159 / 271), 2D 1024 1.01 (106 / 97, 108 / 120; 2048: 0.95), 4D 8192 1.13
+// (154 / 121, 482 / 486); device steps 3D 1024 1.11 (71 / 60, 75 / 77; 2048:
+// 0.99), none in 2D (512: 0.98), 4D 8192 1.05 (104 / 92, 439 / 459). Four
+// features add by four 32-bit atomics and lose in 2D and 3D at once (1024
+// points: 3D 0.97 in a host pass, 168 / 238 clustered, 0.91 in a device step).
 bool sorts(const tmnn_trainer *tr, int n, SortPass pass) {
   if (!tr->d.morton_sort || n <= 1) return false;
   const int dims = tr->d.spatial_dims;
@@ -1362,13 +1362,23 @@ bool sorts(const tmnn_trainer *tr, int n, SortPass pass) {
     return n > (dims == 2 ? 1 << 15 : (1 << 17) - 1);
   if (dims == 4) return n > 8192;
   if (tr->d.features_per_level == 4) return true;
-  if (pass == kSortHostPass) return n > (dims == 2 ? 2048 : 4096);
+  if (pass == kSortHostPass) return n > (dims == 2 ? 1024 : 4096);
   return dims == 2 || n > 1024;
 }
 
 // The pass of a step by train_step_device's overlap_sort (2: a host batch).
 SortPass step_sort_pass(int overlap_sort) {
   return overlap_sort == 2 ? kSortHostPass : kSortDeviceStep;
+}
+
+// Whether a sorted step's sort runs on the second stream: not a host step's one
+// kernel (kSmallSortKeys), which costs less than the events; a device step's
+// hides beside the previous step (4096 3D points 74 us a step, on the main
+// stream 82). Feature-tile plans read the batch through the permutation (no
+// gather).
+bool sorts_beside(const tmnn_trainer *tr, int n, int overlap_sort) {
+  return (overlap_sort == 1 || (overlap_sort == 2 && n > kSmallSortKeys)) && tr->train_plan.xmem &&
+         sorts(tr, n, step_sort_pass(overlap_sort));
 }
 
 // Buffers of a batch of n points (order: those of its sort too).
@@ -1714,14 +1724,13 @@ int run_forward_backward(tmnn_trainer *tr, const float *d_pos, const float *d_tg
   // the packed weight image (rebuilt after every Adam step) counts with the sort
   if ((rc = ensure_image(tr, tr->train_plan)) != TMNN_OK) return rc;
   const bool visit = !reduce && visit_pass(tr, n);
-  const bool order = sorts(tr, n, external_grad ? kSortHostPass : step_sort_pass(overlap_sort));
-  if (overlap_sort && order && tr->train_plan.xmem) {
-    // feature-tile plans read the batch through the permutation (no gather)
+  if (sorts_beside(tr, n, overlap_sort)) {
     rc = sort_batch_overlapped(tr, d_pos, n, overlap_sort > 1, visit, &perm);
   } else {
     if (visit) rc = launch_visit(tr, d_pos, n, tr->ctx->stream);
     if (rc == TMNN_OK)
-      rc = sort_batch(tr, d_pos, d_tgt, tr->d.num_outputs, n, &pos, &tgt, &perm, order,
+      rc = sort_batch(tr, d_pos, d_tgt, tr->d.num_outputs, n, &pos, &tgt, &perm,
+                      sorts(tr, n, external_grad ? kSortHostPass : step_sort_pass(overlap_sort)),
                       !tr->train_plan.xmem);
   }
   if (rc != TMNN_OK || (rc = prof_mark(tr, 1)) != TMNN_OK) return visit ? visit_drop(tr, rc) : rc;
@@ -1985,8 +1994,7 @@ int train_step_device(tmnn_trainer *tr, const float *d_pos, const float *d_tgt, 
   int rc = prof_begin_step(tr);
   if (rc != TMNN_OK) return rc;
   float *loss = d_loss ? d_loss : tr->loss_out.as<float>();
-  const bool overlapped =
-      overlap_sort && sorts(tr, n, step_sort_pass(overlap_sort)) && tr->train_plan.xmem;
+  const bool overlapped = sorts_beside(tr, n, overlap_sort);
   tr->num_this_step = num;
   tr->input_ready = input_ready;
   const int blocks = run_forward_backward(tr, d_pos, d_tgt, n, false, loss, false, overlap_sort);
