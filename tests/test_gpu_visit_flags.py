@@ -73,9 +73,12 @@ def test_visited_entries_are_the_corners(dims, feats, log2t, levels, n):
             assert np.array_equal(moved, want)
 
 
-@pytest.mark.parametrize("dims,feats,log2t,levels,n", [
-    (3, 2, 14, 16, 524288), (3, 4, 17, 8, 262149), (4, 2, 16, 8, 131073), (3, 1, 15, 5, 262201)])
-def test_gradients_match_the_split_path(dims, feats, log2t, levels, n):
+# the last two: level slices above 8 MB, where the split path's backward goes
+# level by level
+@pytest.mark.parametrize("dims,feats,log2t,levels,n,base", [
+    (3, 2, 14, 16, 524288, 16.0), (3, 4, 17, 8, 262149, 16.0), (4, 2, 16, 8, 131073, 16.0),
+    (3, 1, 15, 5, 262201, 16.0), (3, 4, 21, 2, 262145, 128.0), (4, 2, 22, 2, 131073, 64.0)])
+def test_gradients_match_the_split_path(dims, feats, log2t, levels, n, base):
     """One fused step against forward_for_training, backward_accumulate (which
     stores its flags in the backward) and adam_step: first moments within 16
     fixed-point units times 1 - beta1, as the parity tests allow for an ulp of
@@ -85,7 +88,7 @@ def test_gradients_match_the_split_path(dims, feats, log2t, levels, n):
     pos = _positions(dims, n, rng)
     tgt = rng.random((n, 2), dtype=np.float32) * np.float32(200.0)  # large gradients
     enc = dict(n_levels=levels, n_features_per_level=feats, log2_hashmap_size=log2t,
-               base_resolution=16.0, per_level_scale=1.5)
+               base_resolution=base, per_level_scale=1.5)
     args = (dims, 2, enc, dict(n_neurons=64, n_hidden_layers=1))
     kw = dict(loss="L2", precision="fp32", batch=n, hash_range=0.5)
     with make_trainer(*args, **kw) as a, make_trainer(*args, **kw) as b:
